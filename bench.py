@@ -103,7 +103,7 @@ def attainable_mfma(achieved: float) -> dict:
     """The dense int8 MFMA rate this MI355X sustains with random operand bytes
     (the statistics of residue planes), measured after the timed region by
     rns8_amd/probe/librns8_probe.so: every CU issuing back-to-back
-    v_mfma_i32_32x32x32_i8 from registers, ~50 ms so the power controller has
+    v_mfma_i32_16x16x64_i8 from registers, ~50 ms so the power controller has
     settled. The chip is power-limited on such operands, so this, not the
     5.0 POP/s peak, is the ceiling a GEMM on this data can approach; zero
     operands are measured beside it for the clock contrast."""
@@ -126,7 +126,7 @@ def attainable_mfma(achieved: float) -> dict:
         f"{zg:.3f} GHz")
     return {"value": round(rt, 1), "unit": "TOP/s", "clock_ghz": round(rg, 3), "frac": round(achieved / rt, 4),
             "zero_operands": {"value": round(zt, 1), "clock_ghz": round(zg, 3)},
-            "source": "rns8_amd/probe: back-to-back v_mfma_i32_32x32x32_i8 on every CU with random int8 "
+            "source": "rns8_amd/probe: back-to-back v_mfma_i32_16x16x64_i8 on every CU with random int8 "
                       "operands, measured after the timed region"}
 
 
@@ -370,16 +370,16 @@ def main() -> int:
     if tiled:
         workload = (f"RNS8_BOUNDED_I64 {M}x{N}x{K}, per-tile bounds ({tile}x{tile} tiles, A tile rows at "
                     f"2^{TILED_ROW_BITS} cycling, B at 2^{bits}), storage prefix {P}, pack+GEMM+Garner device-resident")
-        kernel = "plane_gemm_kernel<Cfg<4,4>,1,true,true,false> (listed 256x256 units, persistent)"
+        kernel = "plane_gemm_kernel<Cfg<8,8,2>,1,true,false> (listed 256x256 units, persistent)"
     elif args.config == "c3":
         workload = f"RNS8_BOUNDED_I64 {M}x{N}x{K} prefix {P} (FORCE_FIXED_PREFIX), pack+GEMM+Garner device-resident"
-        kernel = "plane_gemm_kernel<Cfg<4,4>,1,true,false,false> (256x256 tiles, persistent)"
+        kernel = "plane_gemm_kernel<Cfg<8,8,2>,1,false,false> (256x256 tiles, persistent)"
     elif args.config == "c5":
         workload = f"c5 {sem} {M}x{N}x{K} prefix {P}, pack+GEMM+Garner device-resident"
-        kernel = "plane_gemm_kernel<Cfg<2,2>,2,true,false,false> K split + residue_finalize_kernel"
+        kernel = "plane_gemm_kernel K split + residue_finalize_kernel"
     else:
         workload = f"{args.config} {sem} {M}x{N}x{K} prefix {P}, pack+GEMM+Garner device-resident"
-        kernel = "plane_gemm_kernel<Cfg<2,2>,2,true,false,false> (128x128 tiles, persistent)"
+        kernel = "plane_gemm_kernel (persistent)"
 
     if args.config == "c3":
         metric = "exact int64 GEMM effective TOPS (2MNK/s) at 4096\u00b3 prefix 9; % int8 MFMA peak"
@@ -673,7 +673,7 @@ def grouped_bench(args) -> int:
                    "stage_ms": {"pack": round(stage[0], 4), "grouped_gemm": round(stage[1], 4),
                                 "export": round(stage[2], 4), "ungrouped_gemms": round(ungrouped, 4)},
                    "range_status": int(status[0]), "rows_bit_exact": exact, "settle_steps": args.settle_steps},
-        "roofline": {"bound": "mfma", "kernel": "plane_gemm_kernel<Cfg<4,4>,1,true,false,true> (grouped, persistent)",
+        "roofline": {"bound": "mfma", "kernel": "plane_gemm_kernel<Cfg<8,8,2>,1,false,true> (grouped, persistent)",
                      "achieved": round(achieved, 2), "peak": PEAK_INT8_TOPS, "unit": "TOP/s",
                      "frac": round(achieved / PEAK_INT8_TOPS, 4), "traffic": None, "per_launch_ops": gemm_ops},
         "cpu_baseline": None,
@@ -808,7 +808,7 @@ def finite_or_wide_bench(args) -> int:
                                 "gemm": round(stage[2], 4), "export": round(stage[3], 4)},
                    "range_status": int(status[0]), "sampled_outputs_exact": exact,
                    "settle_steps": args.settle_steps},
-        "roofline": {"bound": "mfma", "kernel": "plane_gemm_kernel<Cfg<4,4>,1,true,false,false> (256x256 tiles, persistent)",
+        "roofline": {"bound": "mfma", "kernel": "plane_gemm_kernel<Cfg<8,8,2>,1,false,false> (256x256 tiles, persistent)",
                      "achieved": round(achieved, 2), "peak": PEAK_INT8_TOPS, "unit": "TOP/s",
                      "frac": round(achieved / PEAK_INT8_TOPS, 4), "traffic": None, "per_launch_ops": ops * P},
         "cpu_baseline": None,

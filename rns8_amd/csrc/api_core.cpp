@@ -736,6 +736,16 @@ rns8_status init_plan(const rns8_gemm_desc& d, rns8_backend_kind backend, rns8_p
   return RNS8_SUCCESS;
 }
 
+static const char* tile_kernel_name(GemmTile t) {
+  switch (t) {
+    case GemmTile::k256x256: return "plane_gemm_kernel 256x256 tile, 4-stage LDS DMA ring";
+    case GemmTile::k256x128: return "plane_gemm_kernel 256x128 tile, 4-stage LDS DMA ring";
+    case GemmTile::k128x256: return "plane_gemm_kernel 128x256 tile, 4-stage LDS DMA ring";
+    case GemmTile::k64x64: return "plane_gemm_kernel 64x64 tile, 4-stage LDS DMA ring";
+    default: return "plane_gemm_kernel 128x128 tile, 4-stage LDS DMA ring";
+  }
+}
+
 }  // namespace rns8x
 
 rns8_status rns8_create_plan(rns8_context* ctx, const rns8_gemm_desc* desc, rns8_plan** out) {
@@ -855,22 +865,21 @@ rns8_status rns8_get_plan_backend_info(const rns8_plan* plan, rns8_plan_backend_
     const bool listed = per_tile(plan->desc.bound_kind) && !plan->schedule.entries.empty();
     const uint32_t planes = uses_finite_storage(plan->desc.semantics) ? 1u : (plan->prefix ? plan->prefix : 1u);
     const GemmShape shape = choose_gemm_shape(plan->desc.m, plan->desc.n, plan->desc.k, planes);
-    const bool skinny = !listed && shape.tile == 16;
+    const bool skinny = !listed && shape.tile == GemmTile::kSkinny;
     copy_text(out->selected_kernel, sizeof(out->selected_kernel),
               listed ? (plan->unit_edge == 256 ? "plane_gemm_kernel listed 256x256 units (per-tile schedule)"
                                                : "plane_gemm_kernel listed 128x128 units (per-tile schedule)")
               : skinny ? (shape.slices > 1 ? "skinny_gemm_kernel 16-column rows, K split + residue_finalize_kernel"
                                            : "skinny_gemm_kernel 16-column rows")
-              : shape.slices > 1 ? "plane_gemm_kernel 128x128 K split + residue_finalize_kernel"
-              : shape.tile == 256 ? "plane_gemm_kernel 256x256 tile, 4-stage LDS DMA ring"
-                                  : "plane_gemm_kernel 128x128 tile, 4-stage LDS DMA ring");
+              : shape.slices > 1 ? "plane_gemm_kernel K split + residue_finalize_kernel"
+              : tile_kernel_name(shape.tile));
     copy_text(out->accelerator_library, sizeof(out->accelerator_library), "none (hand-written HIP)");
     copy_text(out->capability_status, sizeof(out->capability_status), "available");
     copy_text(out->epilogue_mode, sizeof(out->epilogue_mode), "in_register_centered_reduction");
     copy_text(out->workspace_mode, sizeof(out->workspace_mode),
               plan->splitk_slices > 1 ? "splitk_int8_residues" : "none");
     copy_text(out->isa_evidence, sizeof(out->isa_evidence),
-              skinny ? "gfx950 v_mfma_i32_16x16x64_i8" : "gfx950 v_mfma_i32_32x32x32_i8");
+              "gfx950 v_mfma_i32_16x16x64_i8");
     out->accumulator_k_block_size = static_cast<uint64_t>(plan->desc.k < kSafeKBlock ? plan->desc.k : kSafeKBlock);
     out->accumulator_k_block_cap = static_cast<uint64_t>(kSafeKBlock);
     out->accumulator_modulus = uses_finite_storage(plan->desc.semantics) ? plan->desc.finite_modulus : 0;

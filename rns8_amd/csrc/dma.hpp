@@ -56,6 +56,28 @@ __device__ __forceinline__ void dma16(uint32_t lds_addr, uint32_t voffset, v4i r
                : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voffset), "s"(rsrc)
                : "m0");
 }
+// The same to lds_base + 1024 * block (block a constant below 8 once the
+// caller's loop is unrolled): the offset is the addition's literal, so a block
+// costs one scalar instruction beside its load.
+template <int kBlock>
+__device__ __forceinline__ void dma16_at(uint32_t lds_base, uint32_t voffset, v4i rsrc) {
+  asm volatile("s_add_u32 m0, %0, %3\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+               :
+               : "s"(lds_base), "v"(voffset), "s"(rsrc), "i"(1024 * kBlock)
+               : "m0", "scc");
+}
 #pragma clang diagnostic pop
+__device__ __forceinline__ void dma16_block(uint32_t lds_base, int block, uint32_t voffset, v4i rsrc) {
+  switch (block) {
+    case 0: return dma16_at<0>(lds_base, voffset, rsrc);
+    case 1: return dma16_at<1>(lds_base, voffset, rsrc);
+    case 2: return dma16_at<2>(lds_base, voffset, rsrc);
+    case 3: return dma16_at<3>(lds_base, voffset, rsrc);
+    case 4: return dma16_at<4>(lds_base, voffset, rsrc);
+    case 5: return dma16_at<5>(lds_base, voffset, rsrc);
+    case 6: return dma16_at<6>(lds_base, voffset, rsrc);
+    default: return dma16_at<7>(lds_base, voffset, rsrc);
+  }
+}
 
 }  // namespace rns8x

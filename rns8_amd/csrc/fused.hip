@@ -51,6 +51,7 @@ namespace rns8x {
 namespace {
 
 typedef int v2i __attribute__((ext_vector_type(2)));
+typedef int v16i __attribute__((ext_vector_type(16)));
 
 constexpr int kThreads = 1024;                       // sixteen waves, four per SIMD
 constexpr int kTileM = 128;                          // output rows per workgroup

@@ -9,35 +9,45 @@
 //     on). A persistent grid of workgroups (one per resident slot, a
 //     multiple of 8) walks the unit list, each XCD a contiguous share, so the
 //     DMA stream runs on across unit boundaries.
-//   * workgroup = 256 threads (4 wave64s); waves form a 2x2 grid over the
-//     tile. Two tile configurations: 256x256 (128x128 per wave, 16 MFMA
-//     accumulators, one workgroup per CU) for large outputs and 128x128
-//     (64x64 per wave, two workgroups per CU) when 256x256 tiles would leave
-//     CUs idle.
-//   * K is consumed in BK = 64 byte steps through a 4-stage LDS ring. Both
-//     operands go global -> LDS by buffer-load DMA (no VGPR staging): A tiles
-//     (BM x 64, K-contiguous rows) and B tiles (64 x BN, N-contiguous rows,
-//     the layout they have in HBM). The DMA three K steps ahead is in flight
-//     while a step computes, also across the epilogue into the next unit;
-//     one barrier per step.
+//   * workgroup = 4 wave64s (2 for 64x64 tiles) in a 2 x 2 (2 x 1) grid over
+//     the tile. Five tile configurations (256x256, 256x128, 128x256, 128x128,
+//     64x64); choose_tile takes the one predicted fastest.
+//   * K is consumed in steps of 64. Both operands go global -> LDS by
+//     buffer-load DMA (no VGPR staging). A is staged in chunks of two steps
+//     (BM x 128, K-contiguous rows: whole cache lines; 64-byte rows asked the
+//     L2 for every line twice, and the full lines took 2.4% off 4096^3 at
+//     prefix 9), three chunks deep; B in steps (64 x BN, N-contiguous rows,
+//     the layout it has in HBM), four deep. The DMA four steps ahead is in
+//     flight while a step computes, also across the epilogue into the next
+//     unit; one barrier per step.
 //   * A fragments are ds_read_b128 of 16 K-contiguous bytes; B fragments are
 //     gathered K-contiguous from the N-contiguous stage by ds_read_b64_tr_b8
-//     (LDS transpose read), so no transpose runs on the VALU.
+//     (LDS transpose read), so no transpose runs on the VALU. A step's
+//     fragments are read during the step before.
 //   * Stage rows are XOR-swizzled in 16-byte chunks (swizzle applied on the
 //     global-address side of the DMA) so every fragment read is bank-conflict
 //     free.
-//   * MFMA: v_mfma_i32_32x32x32_i8 with the B^T fragment as src0 and the A
+//   * MFMA: v_mfma_i32_16x16x64_i8 with the B^T fragment as src0 and the A
 //     fragment as src1, so each lane ends with 4 consecutive output columns
-//     of one row per register group -> one packed dword store per group.
+//     of one row. What bounds the large products is the power limit: with
+//     random residue bytes the chip sustains 4.08-4.11 POP/s of back-to-back
+//     16x16x64 MFMAs at 2.0 GHz, against 3.38-3.43 POP/s of 32x32x32 ones
+//     (whose accumulator traffic per product is twice as large); with zero
+//     bytes both reach 4.9. At 4096^3, 9 planes, 32x32x32 tiles took 518 us
+//     (2.39 POP/s), this kernel 452 us (2.73) on the same box, at equal cycles
+//     (0.90 -> 0.86 M) and a 15% higher clock. Of its time, copies without
+//     the operand DMA took 358 of 460 us, without the epilogue 415.
 //   * Exactness: |a*b| <= 2^14, so <= 65536 products plus a carried residue
 //     fit int32. One launch covers at most 65536 K; the host issues longer K
 //     as consecutive launches whose epilogues add the residue already in C.
-//   * Epilogue: accumulators start at 2^31, so each holds the biased sum the
-//     reduction reads; reduction is a byte dot product plus a 24-bit
-//     reciprocal quotient (full-rate VALU only); 4 residues are packed per
-//     dword and staged through a per-wave LDS region (outside the stage
-//     ring) into row-contiguous 16-byte stores.
-//   * Split-K (few output tiles, 128x128 tiles): one launch covers the
+//   * Epilogue: accumulators start at kGemmAccBias (an MFMA inline constant:
+//     no accumulator writes), so each holds the biased sum the reduction
+//     reads; reduction is a byte dot product plus a 24-bit reciprocal quotient
+//     (full-rate VALU only); 4 residues are packed per dword, and four blocks'
+//     dwords are transposed across lane groups by half-wave and row swaps
+//     into 16-byte stores. Staging them through LDS instead took 13.2 k
+//     cycles per 256x256 unit against 8.5 k.
+//   * Split-K (few output tiles): one launch covers the
 //     whole K; each slice (at most 65536 K) reduces its tile like an
 //     unsplit unit and stores the centered residues to its own slot of an
 //     int8 workspace; residue_finalize adds the slots and writes C
@@ -46,6 +56,7 @@
 //   * Results at most 16 columns wide run in skinny.hip instead.
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <mutex>
 #include <type_traits>
 
@@ -57,83 +68,71 @@ namespace rns8x {
 namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v16i __attribute__((ext_vector_type(16)));
 typedef int v2i __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) v2i lds_v2i;
 
 __device__ __forceinline__ lds_v2i* as_lds_v2i(const int8_t* p) {
   return (lds_v2i*)(const_cast<int8_t*>(p));  // generic -> LDS address space
 }
-constexpr int kWaitVm[9] = {wait_vm(0), wait_vm(1), wait_vm(2), wait_vm(3), wait_vm(4),
-                            wait_vm(5), wait_vm(6), wait_vm(7), wait_vm(8)};
 
-constexpr int kThreads = 256;
-constexpr int kGroupM = 4;  // tile rows per L2 reuse group
-// Accumulator start value: the MFMAs then produce u = 2^31 + sum (mod 2^32),
-// the biased form the reduction reads (|sum| < 2^31).
-constexpr int kAccBias = static_cast<int>(0x80000000u);
+// Accumulator start value (tables.hpp): the MFMAs then produce u = bias + sum,
+// the non-negative form the reduction reads (|sum| <= 2^30 + 128).
+constexpr int kAccBias = static_cast<int>(kGemmAccBias);
 
-// Tile configuration: each of the 4 waves (a 2 x 2 grid) owns WM x WN blocks
-// of 32 x 32 outputs, so a workgroup tile is (64 WM) x (64 WN). K steps are 64
-// bytes through 4 LDS stages.
-template <int WM, int WN>
+// Tile configuration: kWaves waves (2 x WN) each own TM x TN blocks of 16 x 16
+// outputs, so a workgroup tile is (32 TM) x (16 TN WN). K advances in steps of
+// 64; A is staged in chunks of two steps.
+template <int TM_, int TN_, int WN_>
 struct Cfg {
-  static constexpr int kWM = WM, kWN = WN;
-  static constexpr int BM = 64 * WM, BN = 64 * WN, BK = 64;
-  static constexpr int kBufA = BM * BK;               // A stage: BM rows x 64 bytes
+  static constexpr int TM = TM_, TN = TN_, WN = WN_;
+  static constexpr int kWaves = 2 * WN, kThreads = 64 * kWaves;
+  static constexpr int BM = 32 * TM, BN = 16 * TN * WN, BK = 64;
+  static constexpr int kBufA = BM * 2 * BK;           // A chunk: BM rows x 128 bytes
   static constexpr int kBufB = BK * BN;               // B stage: 64 k-rows x BN bytes
-  static constexpr int kStage = kBufA + kBufB;
-  static constexpr int kStages = 4;
-  static constexpr int kLds = kStages * kStage;
-  static constexpr int kDmaA = kBufA / 4096;          // 1 KB DMA blocks per wave (4 waves)
-  static constexpr int kDmaB = kBufB / 4096;
+  static constexpr int kSlotsA = 3, kStagesB = 4;
+  static constexpr int kLds = kSlotsA * kBufA + kStagesB * kBufB;
+  static constexpr int kDmaA = kBufA / 2048 / kWaves; // 1 KB DMA blocks per wave and step
+  static constexpr int kDmaB = kBufB / 1024 / kWaves;
+  static constexpr int kGroupM = 1024 / BM;           // tile rows per L2 reuse group
   static constexpr int kChunksB = BN / 16;            // 16-byte chunks per B stage row
   static constexpr int kRowsPerBlockB = 1024 / BN;    // k rows per 1 KB B block
-  static constexpr int kEpiRow = 32 * WN;             // bytes of one wave's output row
-  static constexpr int kEpiChunks = kEpiRow / 16;
-  static constexpr int kEpiRowsPerStore = 64 / kEpiChunks;
-  static constexpr int kEpiBytes = 32 * WM * kEpiRow; // one wave's output block
-  // The epilogue stages output through its own LDS region after the stage
-  // ring, in kEpiParts passes (two for 256x256 tiles: 4 waves x 8 KB).
-  static constexpr int kEpiParts = WM >= 4 ? 2 : 1;
-  static constexpr int kEpiLds = 4 * kEpiBytes / kEpiParts;
-  static_assert(kDmaA >= 1 && kDmaB >= 1 && WM % kEpiParts == 0, "tile config");
-  static_assert(kLds + kEpiLds <= 160 * 1024, "LDS per workgroup");
+  static_assert(kDmaA >= 1 && kDmaA <= 4 && kDmaB >= 1 && kDmaB <= 4, "DMA blocks");
+  static_assert(1024 % BN == 0 && TM % 2 == 0 && TN % 4 == 0, "tile config");
+  static_assert(kLds <= 160 * 1024, "LDS per workgroup");
 };
 
-// A stage: row-major BM x 64 bytes. The 16-byte chunk index is XORed with row
-// bits 1-5 so the ds_read_b128 fragment loads (32 consecutive rows, one chunk)
-// are bank-conflict free for both 32-bank/8-lane and 64-bank/16-lane
-// servicing (exhaustive host model).
-__device__ __forceinline__ int swizzle_a(int row, int chunk) {
-  return chunk ^ (((row >> 1) & 3) ^ (((row >> 3) & 1) * 3) ^ ((row >> 4) & 3));
-}
+// A chunk: row-major BM x 128 bytes, whole cache lines of A. The 16-byte chunk
+// index is XORed with f(row) so the ds_read_b128 fragment loads (16
+// consecutive rows, one chunk per 16 lanes) are bank-conflict free for both
+// 32-bank/8-lane servicing (8 consecutive rows get distinct f) and
+// 64-bank/16-lane servicing (the 8 even and the 8 odd of 16 rows each do).
+__device__ __forceinline__ int swizzle_a(int row, int chunk) { return chunk ^ ((row ^ ((row >> 3) & 1)) & 7); }
 
 // B stage: row-major 64 (k) x BN bytes, N-contiguous as in global memory. A
 // 16-lane transpose read touches 8 consecutive k rows of one chunk; the chunk
-// index is XORed with f(k & 7) so those rows (and, in the 64-bank model, the
-// neighbouring group's) land in distinct bank quads: f(x) = 2x mod 16 + x / 4
-// for 16-chunk rows, f(x) = x for 8-chunk rows (exhaustive host model).
+// index is XORed with f(k) so those rows land in distinct bank quads, and bit
+// 4 of k moves the next 16 lanes' rows (k + 16, the same chunk) onto the bank
+// quads the first leave free: f = 2x mod 16 + x / 4 for 16-chunk rows, f = x
+// for 8-chunk ones (x = k mod 8), either XORed with that bit.
 template <int BN>
 __device__ __forceinline__ int swizzle_b(int k, int chunk) {
-  const int x = k & 7;
+  const int x = k & 7, b4 = (k >> 4) & 1;
   if constexpr (BN == 256)
-    return chunk ^ (((2 * x) & 15) | (x >> 2));
+    return chunk ^ ((((2 * x) & 15) | (x >> 2)) ^ b4);
+  else if constexpr (BN == 128)
+    return chunk ^ (x ^ b4);
   else
-    return chunk ^ x;
+    return chunk ^ (((x >> 1) ^ b4) & 3);
 }
 
-
-// Scheduling slots of a K sub-step region: slot Q is one MFMA followed by up
-// to kPerSlot of the region's kReads LDS fragment reads.
-template <int kId, int Q, int kSlots, int kPerSlot, int kReads>
+// Scheduling slots of a half-step region: kPer MFMAs, then one of the region's
+// kReads LDS fragment reads, kReads times.
+template <int kId, int kPer, int kReads>
 __device__ __forceinline__ void sched_slots() {
-  if constexpr (Q < kSlots) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, kId);  // MFMA
-    constexpr int kLeft = kReads - Q * kPerSlot;
-    constexpr int kNum = kLeft < kPerSlot ? kLeft : kPerSlot;
-    if constexpr (kNum > 0) __builtin_amdgcn_sched_group_barrier(0x100, kNum, kId);  // DS read
-    sched_slots<kId, Q + 1, kSlots, kPerSlot, kReads>();
+  if constexpr (kReads > 0) {
+    __builtin_amdgcn_sched_group_barrier(0x008, kPer, kId);  // MFMA
+    __builtin_amdgcn_sched_group_barrier(0x100, 1, kId);     // DS read
+    sched_slots<kId, kPer, kReads - 1>();
   }
 }
 
@@ -149,6 +148,7 @@ struct UnitMap {
   DivU31 rows;    // kGroupM: tile rows of a full group
   DivU31 tail;    // tile rows of the last group (tiles_m - its first row)
   uint32_t k_begin, k_stop, k_slice;
+  uint32_t pairs;  // K chunks (two steps) every unit runs, at least 2; past the slice's K they read zeros
   // listed launches: two words per unit, (plane << 24 | tile row) and
   // (quadrant mask << 24 | tile column), in place of the arithmetic order
   const uint32_t* list;
@@ -169,18 +169,18 @@ using GroupArg = std::conditional_t<kGrouped, TaskTable, NoTaskTable>;
 // floor(n / d) for n < 2^31 (make_div_u31).
 __device__ __forceinline__ uint32_t div_u31(uint32_t n, DivU31 v) { return __umulhi(n << 1, v.mul) >> v.shift; }
 
-template <typename C, int kMinBlocks, bool kUniform, bool kListed = false, bool kGrouped = false>
-__global__ __launch_bounds__(kThreads, kMinBlocks) void plane_gemm_kernel(GemmArgs args, PlaneConsts pc, UnitMap map,
+template <typename C, int kMinBlocks, bool kListed = false, bool kGrouped = false>
+__global__ __launch_bounds__(C::kThreads, kMinBlocks) void plane_gemm_kernel(GemmArgs args, PlaneConsts pc, UnitMap map,
                                                                            uint32_t accumulate,
                                                                            GroupArg<kGrouped> tasks) {
-  constexpr int WM = C::kWM, WN = C::kWN, BM = C::BM, BN = C::BN, BK = C::BK;
-  __shared__ __attribute__((aligned(16))) int8_t lds[C::kLds + C::kEpiLds];
+  constexpr int TM = C::TM, TN = C::TN, BM = C::BM, BN = C::BN, BK = C::BK;
+  __shared__ __attribute__((aligned(16))) int8_t lds[C::kLds];
 
   const int tid = static_cast<int>(threadIdx.x);
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wave_m = wave >> 1;
-  const int wave_n = wave & 1;
+  const int wave_m = wave / C::WN;
+  const int wave_n = wave % C::WN;
 
   // ---- persistent work list ----------------------------------------------------
   // A unit is one (K slice, plane, output tile). The grid holds a few
@@ -208,16 +208,14 @@ __global__ __launch_bounds__(kThreads, kMinBlocks) void plane_gemm_kernel(GemmAr
   u_end = __builtin_amdgcn_readfirstlane(u_end);
 
   // Units are decoded on the scalar unit (every value here is uniform) with
-  // the host's reciprocals, branch-free, so the cursor below can advance
-  // every K step without splitting the loop body.
+  // the host's reciprocals.
   struct Unit {
-    uint32_t task, plane, slice, m0, n0, kbeg, kend, ktiles, quad;
+    uint32_t task, plane, slice, m0, n0, kbeg, kend, quad;
   };
   // Listed units come from a per-tile schedule: a BM x BN tile of one plane
-  // whose four quadrants (one per wave, 2 x 2) are stored only where the mask
-  // has their bit (wave_m * 2 + wave_n); quadrants outside the tiles that
-  // select this plane keep their contents.
-  static_assert(kThreads == 256, "quadrant masks assume four waves in a 2 x 2 grid");
+  // whose four quadrants (2 x 2) are stored only where the mask has their bit
+  // (2 * row half + column half); quadrants outside the tiles that select this
+  // plane keep their contents.
   auto decode = [&](uint32_t u) {
     Unit U;
     U.task = 0;
@@ -234,7 +232,6 @@ __global__ __launch_bounds__(kThreads, kMinBlocks) void plane_gemm_kernel(GemmAr
       U.quad = w1 >> 24;
       U.kbeg = map.k_begin;
       U.kend = map.k_stop;
-      U.ktiles = (U.kend - U.kbeg + BK - 1) / BK;
       return U;
     }
     U.quad = 0xFu;
@@ -243,15 +240,14 @@ __global__ __launch_bounds__(kThreads, kMinBlocks) void plane_gemm_kernel(GemmAr
     U.slice = div_u31(plane_slice, map.planes);
     U.plane = plane_slice - U.slice * map.planes.d;
     const uint32_t group = div_u31(pid, map.group);
-    const uint32_t first_m = group * kGroupM;
+    const uint32_t first_m = group * C::kGroupM;
     const uint32_t rem = pid - group * map.group.d;
-    const DivU31 rows = first_m + kGroupM <= map.tiles_m ? map.rows : map.tail;
+    const DivU31 rows = first_m + C::kGroupM <= map.tiles_m ? map.rows : map.tail;
     const uint32_t tn = div_u31(rem, rows);
     U.m0 = (first_m + rem - tn * rows.d) * BM;
     U.n0 = tn * BN;
     U.kbeg = map.k_begin + U.slice * map.k_slice;
     U.kend = min(map.k_stop, U.kbeg + map.k_slice);
-    U.ktiles = U.kend > U.kbeg ? (U.kend - U.kbeg + BK - 1) / BK : 0u;
     return U;
   };
 
@@ -285,154 +281,142 @@ __global__ __launch_bounds__(kThreads, kMinBlocks) void plane_gemm_kernel(GemmAr
   // resource): they only feed output columns >= ldc, which are never stored.
   const uint32_t lda = static_cast<uint32_t>(args.lda), ldb = static_cast<uint32_t>(args.ldb);
   const uint32_t m_rows = static_cast<uint32_t>(args.m);
-  uint32_t a_voff[C::kDmaA];  // wave w fills A rows [16 kDmaA w, 16 kDmaA (w + 1))
-  uint32_t b_voff[C::kDmaB];  // wave w fills B k rows [kRowsPerBlockB kDmaB w, ...)
+  // Wave w fills the A chunk's blocks (8 rows of 128 bytes) [2 kDmaA w, 2
+  // kDmaA (w + 1)), half of them in each step of the pair, and B k rows
+  // [kRowsPerBlockB kDmaB w, kRowsPerBlockB kDmaB (w + 1)).
+  uint32_t a_voff[2 * C::kDmaA];
+  uint32_t b_voff[C::kDmaB];
 #pragma unroll
-  for (int i = 0; i < C::kDmaA; ++i) {
-    const int row = 16 * (wave * C::kDmaA + i) + (lane >> 2);
-    a_voff[i] = static_cast<uint32_t>(row) * lda + static_cast<uint32_t>(16 * swizzle_a(row, lane & 3));
+  for (int i = 0; i < 2 * C::kDmaA; ++i) {
+    const int row = 8 * (wave * 2 * C::kDmaA + i) + (lane >> 3);
+    a_voff[i] = static_cast<uint32_t>(row) * lda + static_cast<uint32_t>(16 * swizzle_a(row, lane & 7));
   }
 #pragma unroll
   for (int i = 0; i < C::kDmaB; ++i) {
     const int k = C::kRowsPerBlockB * (wave * C::kDmaB + i) + lane / C::kChunksB;
     b_voff[i] = static_cast<uint32_t>(k) * ldb + static_cast<uint32_t>(16 * swizzle_b<BN>(k, lane % C::kChunksB));
   }
-  const uint32_t lds_a = lds_address(lds) + static_cast<uint32_t>(wave * C::kDmaA * 1024);
-  const uint32_t lds_b = lds_address(lds) + static_cast<uint32_t>(C::kBufA + wave * C::kDmaB * 1024);
+  const uint32_t lds_a = lds_address(lds) + static_cast<uint32_t>(wave * 2 * C::kDmaA * 1024);
+  const uint32_t lds_b = lds_address(lds) + static_cast<uint32_t>(C::kSlotsA * C::kBufA + wave * C::kDmaB * 1024);
 
-  // DMA cursor: the (unit, K tile) whose DMA is issued next, three K tiles
-  // ahead of the compute position, and nsrc, its buffer resources. Past the
-  // last unit the resources are empty (every lane reads zero), which keeps
-  // the per-step DMA count and therefore the vmcnt bookkeeping uniform.
-  struct TileSrc {
-    v4i a, b;
+  // DMA cursor: the K chunk whose DMA is issued next, two chunks ahead of the
+  // compute position. Past a slice's K and past the last unit the resources
+  // are empty (every lane reads zero), which keeps the per-step DMA count and
+  // therefore the vmcnt bookkeeping uniform. The cursor steps by additions
+  // and enters the next unit exactly when the compute position is two chunks
+  // from the end of its own: one wave per SIMD issues every instruction, and
+  // the ~45 scalar ones of decoding a unit and rebuilding its resources at
+  // every step left the matrix cores idle meanwhile.
+  struct Cursor {
+    const int8_t *a, *b;
+    int32_t a_n;    // bytes of A from `a` to the end of the unit's valid rows (< 2^31: gemm_args_ok)
+    int32_t b_rem;  // k rows left in the unit
+    uint32_t b_n0;  // the unit's column offset
+    int32_t dec;    // 2 BK, or 0 past the last unit (a_n and b_rem stay 0)
   };
-  uint32_t du = u_first, dkt = 0;
-  Unit dU = decode(u_first);
-  TileSrc nsrc;
-  auto cursor_load = [&]() {
-    const bool live = du < u_end;
-    const uint32_t k0 = dU.kbeg + dkt * BK;
-    const uint32_t a_rows = min(static_cast<uint32_t>(BM), m_rows - dU.m0);
-    const uint32_t b_rows = min(static_cast<uint32_t>(BK), dU.kend - k0);
-    const int8_t* const a_panel = base_a(dU) + static_cast<uint64_t>(dU.plane) * args.pitch_a +
-                                  static_cast<uint64_t>(dU.m0) * lda;
-    const int8_t* const b_slab = base_b(dU) + static_cast<uint64_t>(dU.plane) * args.pitch_b +
-                                 static_cast<uint64_t>(k0) * ldb + dU.n0;
-    nsrc = TileSrc{buffer_rsrc(a_panel + k0, live ? a_rows * lda - k0 : 0u),
-                   buffer_rsrc(b_slab, live ? b_rows * ldb - dU.n0 : 0u)};
+  auto cursor_of = [&](const Unit& U, bool live) {
+    const uint32_t a_rows = min(static_cast<uint32_t>(BM), m_rows - U.m0);
+    Cursor c;
+    c.a = base_a(U) + static_cast<uint64_t>(U.plane) * args.pitch_a + static_cast<uint64_t>(U.m0) * lda + U.kbeg;
+    c.b = base_b(U) + static_cast<uint64_t>(U.plane) * args.pitch_b + static_cast<uint64_t>(U.kbeg) * ldb + U.n0;
+    c.a_n = live ? static_cast<int32_t>(a_rows * lda - U.kbeg) : 0;
+    c.b_rem = live ? static_cast<int32_t>(U.kend - U.kbeg) : 0;
+    c.b_n0 = live ? U.n0 : 0u;
+    c.dec = live ? 2 * BK : 0;
+    return c;
   };
-  // General advance: decodes the cursor's unit at every step (the prologue,
-  // and launches whose units differ in K tiles). With uniform units
-  // (kUniform) the cursor crosses exactly one unit boundary per compute unit
-  // (it advances one unit's K tiles per unit), so the unit after the
-  // cursor's is decoded once per compute unit (next_du) and the per-step
-  // advance is only selects: decoding at every step cost ~4% of the kernel.
-  Unit nU = dU;
-  auto cursor_advance = [&](auto uniform) {
-    constexpr bool kFast = decltype(uniform)::value;
-    const bool next_unit = dkt + 1 >= dU.ktiles;
-    du = next_unit ? min(du + u_step, u_end) : du;
-    dkt = next_unit ? 0u : dkt + 1;
-    if constexpr (!kFast) nU = decode(min(du, u_end - 1));
-    if (next_unit) dU = nU;
-    cursor_load();
+  Cursor cur = cursor_of(decode(u_first), u_first < u_end);
+  const uint64_t b_step = static_cast<uint64_t>(BK) * ldb;
+  auto src_a = [&]() { return buffer_rsrc(cur.a, cur.a_n); };
+  auto src_b = [&](int half) {
+    const int32_t rows = min(max(cur.b_rem - half * BK, 0), static_cast<int32_t>(BK));
+    return buffer_rsrc(cur.b + (half ? b_step : 0u),
+                       max(rows * static_cast<int32_t>(ldb) - static_cast<int32_t>(cur.b_n0), 0));
   };
-  // (past the last unit any decoded unit will do: the resources are empty)
-  auto next_du = [&]() { nU = decode(min(du + u_step, u_end - 1)); };
-  cursor_load();
-  auto dma_a = [&](const TileSrc& src, int stage, int i) {
-    dma16(lds_a + static_cast<uint32_t>(stage * C::kStage + 1024 * i), a_voff[i], src.a);
+  auto cursor_advance = [&]() {
+    cur.a += 2 * BK;
+    cur.b += 2 * b_step;
+    cur.a_n = max(cur.a_n - cur.dec, 0);
+    cur.b_rem = max(cur.b_rem - cur.dec, 0);
   };
-  auto dma_b = [&](const TileSrc& src, int stage, int i) {
-    dma16(lds_b + static_cast<uint32_t>(stage * C::kStage + 1024 * i), b_voff[i], src.b);
+  auto dma_a = [&](v4i src, uint32_t slot, int half, int i) {
+    dma16_block(__builtin_amdgcn_readfirstlane(lds_a + slot), half * C::kDmaA + i, a_voff[half * C::kDmaA + i], src);
   };
-  auto issue_next = [&](int stage) {
-#pragma unroll
-    for (int i = 0; i < C::kDmaA; ++i) dma_a(nsrc, stage, i);
-#pragma unroll
-    for (int i = 0; i < C::kDmaB; ++i) dma_b(nsrc, stage, i);
-    cursor_advance(std::false_type{});
+  auto dma_b = [&](v4i src, uint32_t stage, int i) {
+    dma16_block(__builtin_amdgcn_readfirstlane(lds_b + stage), i, b_voff[i], src);
   };
 
   // ---- fragments -------------------------------------------------------------
-  // K sub-step s covers k = 32s .. 32s+31 of a stage; lane l takes the 16 k
-  // values 32s + 16*(l >> 5) + 0..15 for both operands.
-  // A (MFMA src1): lane l holds row l & 31 of a 32-row block: one ds_read_b128.
-  // B (MFMA src0): lane l holds column l & 31 of a 32-column block, gathered
-  // by two ds_read_b64_tr_b8. In each 16-lane group, lane j addresses the
+  // One MFMA covers a whole K step: lane l takes the 16 k values 16*(l >> 4) +
+  // 0..15 of the stage for both operands.
+  // A (MFMA src1): lane l holds row l & 15 of a 16-row block: one ds_read_b128.
+  // B (MFMA src0): lane l holds column l & 15 of a 16-column block, gathered
+  // by two ds_read_b64_tr_b8. In each 16-lane group g, lane j addresses the
   // 8-byte row segment (k = base + (j >> 1), columns 8*(j & 1) .. +7 of the
-  // group's 16 columns) and lane i receives byte i & 7 of the segments of
-  // lanes 2b + (i >> 3), b = 0..7: its column across 8 consecutive k.
-  const int frag_row = lane & 31;
-  const int frag_half = lane >> 5;
-  const int tr_j = lane & 15;
-  const int tr_g = lane >> 4;
+  // block) and lane i receives byte i & 7 of the segments of lanes
+  // 2b + (i >> 3), b = 0..7: its column across 8 consecutive k.
+  const int frag_row = lane & 15;
+  const int frag_k = lane >> 4;
   struct Frags {
-    v4i a[WM];
-    v4i b[WN];
+    v4i a[TM];
+    v4i b[TN];
   };
-  auto read_a = [&](int stage, int s, int i) {
-    const int r = wave_m * (32 * WM) + 32 * i + frag_row;
-    return *reinterpret_cast<const v4i*>(lds + stage * C::kStage + r * BK + swizzle_a(r, 2 * s + frag_half) * 16);
+  // (slots and stages are byte offsets)
+  auto read_a = [&](uint32_t slot, int half, int i) {
+    const int r = wave_m * (16 * TM) + 16 * i + frag_row;
+    return *reinterpret_cast<const v4i*>(lds + slot + r * (2 * BK) + swizzle_a(frag_row, 4 * half + frag_k) * 16);
   };
-  auto read_b = [&](int stage, int s, int j) {
-    const int8_t* const sb = lds + stage * C::kStage + C::kBufA;
-    const int ncol = wave_n * (32 * WN) + 32 * j + 16 * (tr_g & 1) + 8 * (tr_j & 1);
-    const int k = 32 * s + 16 * (tr_g >> 1) + (tr_j >> 1);
-    const v2i lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
-        as_lds_v2i(sb + k * BN + swizzle_b<BN>(k, ncol >> 4) * 16 + (ncol & 8)));
-    const v2i hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
-        as_lds_v2i(sb + (k + 8) * BN + swizzle_b<BN>(k + 8, ncol >> 4) * 16 + (ncol & 8)));
+  auto read_b = [&](uint32_t stage, int j) {
+    const int8_t* const sb = lds + C::kSlotsA * C::kBufA + stage;
+    const int chunk = wave_n * TN + j;
+    const int k = 16 * frag_k + (frag_row >> 1);
+    const int8_t* const at = sb + k * BN + swizzle_b<BN>(k, chunk) * 16 + 8 * (frag_row & 1);
+    const v2i lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32(as_lds_v2i(at));
+    const v2i hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32(as_lds_v2i(at + 8 * BN));  // f(k + 8) = f(k)
     return v4i{lo[0], lo[1], hi[0], hi[1]};
   };
-  auto read_frags = [&](int stage, int s, Frags& f) {
-#pragma unroll
-    for (int i = 0; i < WM; ++i) f.a[i] = read_a(stage, s, i);
-#pragma unroll
-    for (int j = 0; j < WN; ++j) f.b[j] = read_b(stage, s, j);
-  };
 
-  v16i acc[WM][WN];
-  auto reset_acc = [&]() {
+  v4i acc[TM][TN];
+  // The MFMAs of block rows [i0, i0 + TM/2) for one K step, columns in
+  // alternating order so consecutive MFMAs share an operand. A unit's first
+  // step starts from the bias (an inline constant, no accumulator writes).
+  auto mfma_half = [&](auto first, const Frags& f, int i0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < WM; ++i)
+    for (int ii = 0; ii < TM / 2; ++ii)
 #pragma unroll
-      for (int j = 0; j < WN; ++j) acc[i][j] = v16i{} + kAccBias;
+      for (int jj = 0; jj < TN; ++jj) {
+        const int i = i0 + ii, j = (ii & 1) ? TN - 1 - jj : jj;
+        const v4i start = {kAccBias, kAccBias, kAccBias, kAccBias};
+        acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(f.b[j], f.a[i], decltype(first)::value ? start : acc[i][j],
+                                                          0, 0, 0);
+      }
   };
-  auto mfma_all = [&](const Frags& f) {
-#pragma unroll
-    for (int i = 0; i < WM; ++i)
-#pragma unroll
-      for (int j = 0; j < WN; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f.b[j], f.a[i], acc[i][j], 0, 0, 0);
-  };
-  // Interleave a region's WM*WN MFMAs with its WM + 2*WN fragment reads: the
-  // reads go between the first three quarters of the MFMAs.
-  constexpr int kMfma = WM * WN;
-  constexpr int kReads = WM + 2 * WN;
-  constexpr int kSlots = kMfma - kMfma / 4;
-  constexpr int kPerSlot = (kReads + kSlots - 1) / kSlots;
+  // Interleave a half step's TM/2*TN MFMAs with half of the next position's
+  // fragment reads, spread over its first three quarters.
+  constexpr int kMfma = TM / 2 * TN;
+  constexpr int kReads = TM / 2 + TN;
+  constexpr int kPerSlot = kMfma * 3 / 4 / kReads > 0 ? kMfma * 3 / 4 / kReads : 1;
   // The MFMA builtins carry no ordering of their own, so instruction
   // selection may place some of a region's MFMAs after its sched_barrier; an
   // empty asm statement that takes every accumulator (and is ordered before
   // the barrier) keeps them all inside the region.
-  auto schedule_region = [&](auto id) {
+  auto schedule_region = [&](auto id, int i0) __attribute__((always_inline)) {
     constexpr int kId = decltype(id)::value;
 #pragma unroll
-    for (int i = 0; i < WM; ++i)
+    for (int i = 0; i < TM / 2; ++i)
 #pragma unroll
-      for (int j = 0; j < WN; ++j) asm volatile("" ::"a"(acc[i][j]));
-    sched_slots<kId, 0, kSlots, kPerSlot, kReads>();
-    __builtin_amdgcn_sched_group_barrier(0x008, kMfma - kSlots, kId);
+      for (int j = 0; j < TN; ++j) asm volatile("" ::"a"(acc[i0 + i][j]));
+    sched_slots<kId, kPerSlot, kReads>();
+    if constexpr (kMfma > kPerSlot * kReads)
+      __builtin_amdgcn_sched_group_barrier(0x008, kMfma - kPerSlot * kReads, kId);
     __builtin_amdgcn_sched_barrier(0);
   };
-  constexpr int kRegionLen = (WM > WN ? WM : WN) > C::kDmaA ? (WM > WN ? WM : WN) : C::kDmaA;
 
   // ---- epilogue ---------------------------------------------------------------
-  // acc[i][j] register 4g+e holds u = 2^31 + C[row][col] (mod 2^32; the
-  // accumulators start at 2^31) with
-  //   row = m0 + wave_m*32*WM + 32i + (lane & 31)
-  //   col = n0 + wave_n*32*WN + 32j + 8g + 4*(lane >> 5) + e.
+  // acc[i][j] register e holds u = kAccBias + C[row][col] (the accumulators
+  // start at kAccBias) with
+  //   row = m0 + wave_m*16*TM + 16i + (lane & 15)
+  //   col = n0 + wave_n*16*TN + 16j + 4*(lane >> 4) + e.
   // Stores go through a buffer resource over the unit's tile rows, so rows
   // >= M are dropped by the range check; columns past the padded pitch (only
   // in the last tile column) get an offset beyond num_records.
@@ -444,11 +428,11 @@ __global__ __launch_bounds__(kThreads, kMinBlocks) void plane_gemm_kernel(GemmAr
     const ModulusConsts mc = pc.mod[U.plane];
     const int64_t tile_rows = min(static_cast<int64_t>(BM), args.m - U.m0);
     const uint32_t lane_off =
-        static_cast<uint32_t>((wave_m * (32 * WM) + frag_row) * args.ldc + wave_n * (32 * WN) + 4 * frag_half);
-    const uint32_t row_step = static_cast<uint32_t>(32 * args.ldc);
+        static_cast<uint32_t>((wave_m * (16 * TM) + frag_row) * args.ldc + wave_n * (16 * TN));
+    const uint32_t row_step = static_cast<uint32_t>(16 * args.ldc);
     const bool full_cols = U.n0 + BN <= args.ldc;
     // a listed unit's wave stores its quadrant only if the mask selects it
-    if (kListed && ((U.quad >> (wave_m * 2 + wave_n)) & 1u) == 0u) return;
+    if (kListed && ((U.quad >> (wave_m * 2 + (wave_n >= C::WN / 2 ? 1 : 0))) & 1u) == 0u) return;
     // the unit's tile of C, or of its K slice's workspace slot
     // [slice][plane][M][ldc] (split launches never accumulate)
     int8_t* const Cp =
@@ -457,163 +441,183 @@ __global__ __launch_bounds__(kThreads, kMinBlocks) void plane_gemm_kernel(GemmAr
             : base_ws(U) + ((static_cast<int64_t>(U.slice) * args.nplanes + U.plane) * args.m + U.m0) * args.ldc +
                   U.n0;
     const __amdgpu_buffer_rsrc_t c_rsrc = make_rsrc(Cp, tile_rows * args.ldc - U.n0);
-    const CenteredI32 kc = centered_i32_consts(mc);
-    // The packed residues go through this wave's slice of the epilogue LDS
-    // region (outside the stage ring, so the next unit's DMAs keep landing)
-    // so the global stores are row-contiguous 16-byte chunks; kEpiParts
-    // passes of WM / kEpiParts block rows each. Layout: row-major
-    // kEpiRow-byte rows, 16-byte chunk c of row r at c ^ ((r >> 1) &
-    // (kEpiChunks - 1)).
-    int8_t* const ep = lds + C::kLds + wave * (C::kEpiBytes / C::kEpiParts);
-    auto epi_swz = [](int r) { return (r >> 1) & (C::kEpiChunks - 1); };
-    const int rrow = lane / C::kEpiChunks;
-    const int rchunk = lane % C::kEpiChunks;
-    const bool chunk_ok = full_cols || wave_n * (32 * WN) + 16 * rchunk < static_cast<int>(args.ldc - U.n0);
-    constexpr int kPartRows = WM / C::kEpiParts;  // 32-row blocks per pass
+    const CenteredI32 kc = centered_acc_consts(mc);
+    // Each lane's packed dword of block (i, j) holds 4 columns of a row. Four
+    // neighbouring blocks' dwords are transposed across the four 16-lane
+    // groups (two half-wave and two row swaps), so lane group g holds the 16
+    // bytes of block 4q + g's row and one 16-byte store covers 64 contiguous
+    // bytes of each of 16 rows.
+    auto reduce = [&](auto carry, auto low_byte) {
+      constexpr bool kCarry = decltype(carry)::value;
+      constexpr bool kLowByte = decltype(low_byte)::value;  // m = 256: the residue is the low byte
 #pragma unroll
-    for (int part = 0; part < C::kEpiParts; ++part) {
-      auto reduce = [&](auto carry, auto low_byte) {
-        constexpr bool kCarry = decltype(carry)::value;
-        constexpr bool kLowByte = decltype(low_byte)::value;  // m = 256: the residue is the low byte
+      for (int i = 0; i < TM; ++i) {
+        const uint32_t off = lane_off + static_cast<uint32_t>(i) * row_step;
+        uint32_t prev[TN];
+        if constexpr (kCarry) {
+          // later K block: add the centered residue carried in C (|.| <= 128)
 #pragma unroll
-        for (int ii = 0; ii < kPartRows; ++ii) {
-          const int i = part * kPartRows + ii;
-          const uint32_t off = lane_off + static_cast<uint32_t>(i) * row_step;
-          uint32_t prev[WN][4];
-          if constexpr (kCarry) {
-            // later K block: add the centered residue carried in C (|.| <= 128)
+          for (int j = 0; j < TN; ++j)
+            prev[j] = static_cast<uint32_t>(
+                __builtin_amdgcn_raw_buffer_load_b32(c_rsrc, static_cast<int>(off + 16 * j + 4 * frag_k), 0, 0));
+        }
 #pragma unroll
-            for (int j = 0; j < WN; ++j)
+        for (int q = 0; q < TN / 4; ++q) {
+          uint32_t d[4];
 #pragma unroll
-              for (int g = 0; g < 4; ++g)
-                prev[j][g] = static_cast<uint32_t>(
-                    __builtin_amdgcn_raw_buffer_load_b32(c_rsrc, static_cast<int>(off + 32 * j + 8 * g), 0, 0));
-          }
-          const int r = 32 * ii + frag_row;
-#pragma unroll
-          for (int j = 0; j < WN; ++j) {
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
+          for (int jj = 0; jj < 4; ++jj) {
+            const int j = 4 * q + jj;
+            const Acc4 a4 = acc_read4(acc[i][j]);
+            if constexpr (kLowByte) {
+              // the bias is 0 mod 256, so u's low byte is C's, read as int8 its centered residue
+              d[jj] = pack_low_bytes(a4.v[0], a4.v[1], a4.v[2], a4.v[3]);
+            } else {
               uint32_t res[4];
-              const Acc4 a4 = acc_read4(acc[i][j], g);
-              uint32_t packed;
-              if constexpr (kLowByte) {
-                // 2^31 is 0 mod 256, so u's low byte is C's, read as int8 its centered residue
-                packed = pack_low_bytes(a4.v[0], a4.v[1], a4.v[2], a4.v[3]);
-              } else {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                  uint32_t u = a4.v[e];
-                  if constexpr (kCarry)
-                    u += static_cast<uint32_t>(static_cast<int32_t>(static_cast<int8_t>(prev[j][g] >> (8 * e))));
-                  res[e] = centered_residue_i32(u, mc, kc);
-                }
-                packed = pack_low_bytes(res[0], res[1], res[2], res[3]);
+              for (int e = 0; e < 4; ++e) {
+                uint32_t u = a4.v[e];
+                if constexpr (kCarry)
+                  u += static_cast<uint32_t>(static_cast<int32_t>(static_cast<int8_t>(prev[j] >> (8 * e))));
+                res[e] = centered_residue_i32(u, mc, kc);
               }
-              const int c = 2 * j + (g >> 1);
-              *reinterpret_cast<uint32_t*>(ep + r * C::kEpiRow + ((c ^ epi_swz(r)) << 4) + 8 * (g & 1) +
-                                           4 * frag_half) = packed;
+              d[jj] = pack_low_bytes(res[0], res[1], res[2], res[3]);
             }
           }
+          const auto s02 = __builtin_amdgcn_permlane32_swap(d[0], d[2], false, false);
+          const auto s13 = __builtin_amdgcn_permlane32_swap(d[1], d[3], false, false);
+          const auto t01 = __builtin_amdgcn_permlane16_swap(s02[0], s13[0], false, false);
+          const auto t23 = __builtin_amdgcn_permlane16_swap(s02[1], s13[1], false, false);
+          const v4i v = {static_cast<int>(t01[0]), static_cast<int>(t01[1]), static_cast<int>(t23[0]),
+                         static_cast<int>(t23[1])};
+          const int col = wave_n * (16 * TN) + 64 * q + 16 * frag_k;
+          const bool ok = full_cols || col < static_cast<int>(args.ldc - U.n0);
+          __builtin_amdgcn_raw_buffer_store_b128(
+              v, c_rsrc, static_cast<int>(ok ? off + 64 * q + 16 * frag_k : 0x80000000u), 0, 0);
         }
-      };
-      if (accumulate)
-        reduce(std::true_type{}, std::false_type{});
-      else if (mc.m == 256u)
-        reduce(std::false_type{}, std::true_type{});
-      else
-        reduce(std::false_type{}, std::false_type{});
-      // Read back row-contiguous: lane l takes chunk l % kEpiChunks of rows
-      // q * kEpiRowsPerStore + l / kEpiChunks of this pass.
-      const uint32_t goff = static_cast<uint32_t>((wave_m * (32 * WM) + 32 * kPartRows * part + rrow) * args.ldc +
-                                                  wave_n * (32 * WN) + 16 * rchunk);
-#pragma unroll
-      for (int q = 0; q < 32 * kPartRows / C::kEpiRowsPerStore; ++q) {
-        const int row = C::kEpiRowsPerStore * q + rrow;
-        const v4i v = *reinterpret_cast<const v4i*>(ep + row * C::kEpiRow + ((rchunk ^ epi_swz(row)) << 4));
-        const uint32_t o = goff + static_cast<uint32_t>(C::kEpiRowsPerStore * q) * static_cast<uint32_t>(args.ldc);
-        __builtin_amdgcn_raw_buffer_store_b128(v, c_rsrc, static_cast<int>(chunk_ok ? o : 0x80000000u), 0, 0);
       }
-    }
+    };
+    if (accumulate)
+      reduce(std::true_type{}, std::false_type{});
+    else if (mc.m == 256u)
+      reduce(std::false_type{}, std::true_type{});
+    else
+      reduce(std::false_type{}, std::false_type{});
   };
 
   // ---- pipeline ----------------------------------------------------------------
-  // Four LDS stages. Stream position s (the s-th K tile of this workgroup's
-  // work list, across unit boundaries) is computed from stage s%4 while the
-  // DMA of position s+3 into stage (s+3)%4 (last read at position s-1) is in
-  // flight and the first fragments of position s+1 are prefetched. Before the
-  // barrier that ends position s each wave waits until only its position s+3
-  // DMAs are outstanding (older VMEM operations, the previous epilogue's
-  // stores included, complete in order before them), so the barrier publishes
-  // position s+2 and retires every read of stage s%4. The DMAs are issued
-  // from inline asm, so the compiler tracks no LDS write for them and adds no
-  // waits before the fragment reads: the explicit vmcnt waits below are what
-  // orders them. They are spread over the whole step (A DMAs in the first
-  // half, B DMAs in the second): each one holds the texture path for a while,
-  // and bunching a step's DMAs stalls MFMA issue.
+  // Three A slots (a chunk of two K steps each) and four B stages. Stream
+  // position s (the s-th K step of this workgroup's work list, across unit
+  // boundaries; position s belongs to chunk s / 2) is computed from registers:
+  // its fragments were read during position s-1. While it computes, the
+  // fragments of position s+1 are read, the DMA of B's position s+4 goes into
+  // stage s % 4 and half of A's chunk s/2 + 2 into slot (s/2 + 2) % 3; every
+  // wave finished reading both before the last barrier (B's position s was
+  // read during s-1, chunk s/2 - 1 during at most s-2). Before the barrier
+  // that ends position s each wave waits for its DMAs of position s+2, read
+  // next (issued up to position s-2, or, for the second half of an A chunk,
+  // first in position s-1: then only that position's B DMAs and position s's
+  // may be outstanding; older VMEM operations, the previous epilogue's stores
+  // included, complete in order before them) and for its fragment reads, so
+  // the barrier publishes position s+2 and retires every read of position
+  // s+1. The DMAs are issued from inline asm, so the compiler tracks no LDS
+  // write for them and adds no waits before the fragment reads: the explicit
+  // vmcnt waits below are what orders them. They are spread over the step (A
+  // DMAs in the first half, B DMAs in the second): each one holds the texture
+  // path for a while, and bunching a step's DMAs stalls MFMA issue.
   if (u_first >= u_end) return;
-  constexpr int kDmaPerTile = C::kDmaA + C::kDmaB;
-  Frags f0, f1, f0n;
-  issue_next(0);
-  issue_next(1);
-  issue_next(2);
-  __builtin_amdgcn_s_waitcnt(kWaitVm[kDmaPerTile]);  // positions 0 and 1 landed
+  constexpr int kDmaStep = C::kDmaA + C::kDmaB;
+  Frags f0, f1;
+  uint32_t slot0 = 0, slot1 = C::kBufA, slot2 = 2 * C::kBufA;  // chunks c, c+1, c+2 of the compute position
+  uint32_t stage0 = 0, stage2 = 2 * C::kBufB;                  // B stages of the pair and of the next pair
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const v4i sa = src_a();
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      const v4i sb = src_b(half);
+#pragma unroll
+      for (int i = 0; i < C::kDmaA; ++i) dma_a(sa, c * C::kBufA, half, i);
+#pragma unroll
+      for (int i = 0; i < C::kDmaB; ++i) dma_b(sb, (2 * c + half) * C::kBufB, i);
+    }
+    cursor_advance();
+  }
+  __builtin_amdgcn_s_waitcnt(wait_vm(2 * kDmaStep));  // chunk 0 landed
   __syncthreads();
-  read_frags(0, 0, f0);
-  int stage = 0;
+#pragma unroll
+  for (int i = 0; i < TM; ++i) f0.a[i] = read_a(0, 0, i);
+#pragma unroll
+  for (int j = 0; j < TN; ++j) f0.b[j] = read_b(0, j);
+  __syncthreads();  // B stage 0 is read: position 4 may overwrite it
+  // K step `half` of the pair: MFMAs on `f`, the next position's fragments
+  // into `fn`.
+  auto step = [&](auto first, auto half_c, const Frags& f, Frags& fn) __attribute__((always_inline)) {
+    constexpr int half = decltype(half_c)::value;
+    constexpr int kRegionLen = TM / 2 > TN / 2 ? (TM / 2 > 4 ? TM / 2 : 4) : (TN / 2 > 4 ? TN / 2 : 4);
+    const uint32_t next_slot = half ? slot1 : slot0;
+    const uint32_t next_stage = half ? stage2 : stage0 + C::kBufB;
+    const uint32_t dma_stage = stage0 + half * C::kBufB;
+    const v4i sa = src_a(), sb = src_b(half);
+#pragma unroll
+    for (int t = 0; t < kRegionLen; ++t) {
+      if (t < TM / 2) fn.a[t] = read_a(next_slot, half ^ 1, t);
+      if (t < TN / 2) fn.b[t] = read_b(next_stage, t);
+      if (t < C::kDmaA) dma_a(sa, slot2, half, t);
+    }
+    mfma_half(first, f, 0);
+    schedule_region(std::integral_constant<int, 1>{}, 0);
+#pragma unroll
+    for (int t = 0; t < kRegionLen; ++t) {
+      if (t < TM / 2) fn.a[TM / 2 + t] = read_a(next_slot, half ^ 1, TM / 2 + t);
+      if (t < TN / 2) fn.b[TN / 2 + t] = read_b(next_stage, TN / 2 + t);
+      if (t < C::kDmaB) dma_b(sb, dma_stage, t);
+    }
+    mfma_half(first, f, TM / 2);
+    // the cursor's scalar work issues in the shadow of this region's MFMAs
+    if constexpr (half == 1) cursor_advance();
+    schedule_region(std::integral_constant<int, 2>{}, TM / 2);
+    // the next position's fragments stay in this step
+#pragma unroll
+    for (int i = 0; i < TM; ++i) asm volatile("" ::"v"(fn.a[i]));
+#pragma unroll
+    for (int j = 0; j < TN; ++j) asm volatile("" ::"v"(fn.b[j]));
+    __builtin_amdgcn_s_waitcnt(wait_vm(half ? 2 * kDmaStep : kDmaStep + C::kDmaB));
+    __syncthreads();
+  };
+  auto pair = [&](auto first) __attribute__((always_inline)) {
+    step(first, std::integral_constant<int, 0>{}, f0, f1);
+    step(std::false_type{}, std::integral_constant<int, 1>{}, f1, f0);
+    const uint32_t s = slot0;
+    slot0 = slot1;
+    slot1 = slot2;
+    slot2 = s;
+    stage0 ^= 2 * C::kBufB;
+    stage2 ^= 2 * C::kBufB;
+  };
   for (uint32_t u = u_first; u < u_end; u += u_step) {
     const Unit U = decode(u);
-    if constexpr (kUniform) next_du();
-    reset_acc();
-    // every unit has at least one K tile (the host sizes slices so)
-    uint32_t kt = 0;
-    do {
-      const int stage1 = (stage + 1) & 3;
-      const int stage3 = (stage + 3) & 3;
-      const TileSrc src = nsrc;
-      // Region 1: sub-step 0 MFMAs; sub-step 1 fragment reads and the A DMAs.
-#pragma unroll
-      for (int t = 0; t < kRegionLen; ++t) {
-        if (t < WM) f1.a[t] = read_a(stage, 1, t);
-        if (t < WN) f1.b[t] = read_b(stage, 1, t);
-        if (t < C::kDmaA) dma_a(src, stage3, t);
-      }
-      mfma_all(f0);
-      schedule_region(std::integral_constant<int, 1>{});
-      // Region 2: sub-step 1 MFMAs; first fragments of position s+1 and the B
-      // DMAs.
-#pragma unroll
-      for (int t = 0; t < kRegionLen; ++t) {
-        if (t < WM) f0n.a[t] = read_a(stage1, 0, t);
-        if (t < WN) f0n.b[t] = read_b(stage1, 0, t);
-        if (t < C::kDmaB) dma_b(src, stage3, t);
-      }
-      mfma_all(f1);
-      // The cursor's scalar work sits in this region, where it issues in the
-      // shadow of the MFMAs; after the region it would run with the MFMA
-      // pipe idle.
-      if constexpr (kUniform) cursor_advance(std::true_type{});
-      schedule_region(std::integral_constant<int, 2>{});
-      // the next position's fragments stay in this step (not sunk past the
-      // cursor's branch)
-#pragma unroll
-      for (int i = 0; i < WM; ++i) asm volatile("" ::"v"(f0n.a[i]));
-#pragma unroll
-      for (int j = 0; j < WN; ++j) asm volatile("" ::"v"(f0n.b[j]));
-      if constexpr (!kUniform) cursor_advance(std::false_type{});
-      __builtin_amdgcn_s_waitcnt(kWaitVm[kDmaPerTile]);  // only position s+3 outstanding
-      __syncthreads();
-      f0 = f0n;
-      stage = stage1;
-    } while (++kt < U.ktiles);
+    const Cursor next = cursor_of(decode(min(u + u_step, u_end - 1)), u + u_step < u_end);
+    // The cursor enters the next unit by selects at the pair two chunks
+    // before the end (a branch there makes the compiler duplicate the pair
+    // and spill accumulators).
+    auto enter_next = [&](bool enter) {
+      cur.a = enter ? next.a : cur.a;
+      cur.b = enter ? next.b : cur.b;
+      cur.a_n = enter ? next.a_n : cur.a_n;
+      cur.b_rem = enter ? next.b_rem : cur.b_rem;
+      cur.b_n0 = enter ? next.b_n0 : cur.b_n0;
+      cur.dec = enter ? next.dec : cur.dec;
+    };
+    uint32_t n = map.pairs;
+    enter_next(n == 2u);
+    pair(std::true_type{});
+    for (--n; n; --n) {
+      enter_next(n == 2u);
+      pair(std::false_type{});
+    }
     epilogue(U);
-    // The first fragments of the next unit are read again here rather than
-    // kept from the last step: holding them through the epilogue costs
-    // registers the epilogue needs. The stage stays valid: its next DMA is
-    // issued only in the next step.
-    read_frags(stage, 0, f0);
   }
-  __builtin_amdgcn_s_waitcnt(kWaitVm[0]);  // no DMA outlives the workgroup's LDS
+  __builtin_amdgcn_s_waitcnt(wait_vm(0));  // no DMA outlives the workgroup's LDS
 }
 
 // Zero-output tiles of a per-tile schedule: planes [0, planes) of each tile's
@@ -643,9 +647,11 @@ __global__ __launch_bounds__(256) void zero_words_kernel(uint32_t* dst, uint64_t
     dst[w] = 0u;
 }
 
-using CfgLarge = Cfg<4, 4>;  // 256 x 256 tiles, one workgroup per CU (all 512 registers per lane)
-using CfgSmall = Cfg<2, 2>;  // 128 x 128 tiles, two workgroups per CU
-
+using Cfg256x256 = Cfg<8, 8, 2>;  // one workgroup per CU (all 512 registers per lane)
+using Cfg256x128 = Cfg<8, 4, 2>;  // one per CU (128 KB of LDS)
+using Cfg128x256 = Cfg<4, 8, 2>;  // one per CU (112 KB)
+using Cfg128x128 = Cfg<4, 4, 2>;  // two per CU
+using Cfg64x64 = Cfg<2, 4, 1>;    // two waves, four workgroups per CU
 
 template <typename Cf>
 int64_t tile_count(int64_t m, int64_t n, uint32_t nplanes) {
@@ -654,32 +660,70 @@ int64_t tile_count(int64_t m, int64_t n, uint32_t nplanes) {
 
 }  // namespace
 
+namespace {
+
+// The tile whose launch is predicted fastest. A launch costs a start plus, for
+// the CU with the most units, each unit's K chunks and epilogue (workgroups
+// that share a CU share its matrix cores, so their costs add). The costs, in
+// 10 ns, were fitted to launches of 16 shapes from 256^3 to 4096^3 (K from 256
+// to 30000, 1 to 18 planes; the measured best tile is within 3% of the choice
+// at each). They trade the operand traffic per product (256x256 least) against
+// the units left for the last round: 1024^3 at 9 planes ran 16.7 us with
+// 256x256 tiles (144 units), 18.5 with 256x128, 15.2 with 128x128 (576); 700 x
+// 700 x 3000 at 8 planes 33.0, 20.8, 22.3; one 1024^3 plane 15.6, 9.9, 7.0
+// and 5.6 with 64x64; 4096^3 at 1 plane 52.8, 59.5, 65.0, 128.
+GemmTile choose_tile(int64_t m, int64_t n, int64_t k_slice, int64_t plane_slices) {
+  struct TileCost {
+    GemmTile tile;
+    int64_t bm, bn, start, chunk, unit;
+  };
+  constexpr TileCost kCosts[] = {
+      {GemmTile::k256x256, 256, 256, 400, 150, 300}, {GemmTile::k256x128, 256, 128, 350, 84, 200},
+      {GemmTile::k128x256, 128, 256, 350, 84, 200},  {GemmTile::k128x128, 128, 128, 300, 45, 100},
+      {GemmTile::k64x64, 64, 64, 250, 25, 60}};
+  constexpr int64_t kCus = 256;
+  const int64_t chunks = std::max<int64_t>((std::min<int64_t>(k_slice, kSafeKBlock) + 127) / 128, 2);
+  GemmTile best = GemmTile::k128x128;
+  double best_cost = 0;
+  for (const TileCost& t : kCosts) {
+    const double units = static_cast<double>((m + t.bm - 1) / t.bm) * static_cast<double>((n + t.bn - 1) / t.bn) *
+                         static_cast<double>(plane_slices);
+    if (units > 0x7FFFFFFF) continue;  // unit numbers are 31-bit
+    const double rounds = std::ceil(units / kCus);
+    const double cost = static_cast<double>(t.start) + rounds * static_cast<double>(chunks * t.chunk + t.unit);
+    if (best_cost == 0 || cost < best_cost) {
+      best = t.tile;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
+}  // namespace
+
 GemmShape choose_gemm_shape(int64_t m, int64_t n, int64_t k, uint32_t nplanes) {
   // Results at most 16 columns wide: the skinny kernel (skinny.hip).
   GemmShape shape{};
   if (skinny_shape(m, n, k, nplanes, shape)) return shape;
-  // 256 x 256 tiles when they already give every CU at least one and neither
-  // side of the result is narrower than 256; otherwise 128 x 128 tiles (two
-  // per CU), and split K when even those leave the chip under-filled: toward
-  // ~512 units, with slices of at least 4096 K and at most 65536. Each slice
-  // adds a residue tile per plane to write and sum, and short slices spend a
-  // larger share in the DMA prologue and the epilogue.
-  shape.tile = 128;
+  // K is split when 128 x 128 tiles leave the chip under-filled and K is
+  // long: toward ~512 units of that size, with slices of at least 4096 K and
+  // at most 65536. Each slice adds a residue tile per plane to write and sum,
+  // and short slices spend a larger share in the DMA prologue and the
+  // epilogue.
   shape.slices = 1;
   shape.k_slice = k;
-  if (m > 128 && n > 128 && tile_count<CfgLarge>(m, n, nplanes) >= 256) {
-    shape.tile = 256;
-    return shape;
-  }
-  const int64_t tiles = tile_count<CfgSmall>(m, n, nplanes);
+  shape.tile = choose_tile(m, n, k, nplanes);
+  if (m > 128 && n > 128 && tile_count<Cfg256x256>(m, n, nplanes) >= 256) return shape;
+  const int64_t tiles = tile_count<Cfg128x128>(m, n, nplanes);
   if (tiles >= 256 || k < 8192) return shape;
   int64_t slices = std::min<int64_t>((512 + tiles - 1) / tiles, k / 4096);
   slices = std::max<int64_t>(slices, (k + kSafeKBlock - 1) / kSafeKBlock);
   if (slices <= 1) return shape;
   int64_t k_slice = (k + slices - 1) / slices;
-  k_slice = (k_slice + CfgSmall::BK - 1) / CfgSmall::BK * CfgSmall::BK;
+  k_slice = (k_slice + Cfg128x128::BK - 1) / Cfg128x128::BK * Cfg128x128::BK;
   slices = (k + k_slice - 1) / k_slice;
   if (slices <= 1 || slices * tiles > 0x7FFFFFFF) return shape;
+  shape.tile = choose_tile(m, n, k_slice, nplanes * slices);
   shape.slices = static_cast<uint32_t>(slices);
   shape.k_slice = k_slice;
   shape.ws_bytes = static_cast<uint64_t>(slices) * nplanes * static_cast<uint64_t>(m) * static_cast<uint64_t>(padded_ld(n));
@@ -711,6 +755,10 @@ int device_cu_count() {
   return cus;
 }
 
+// K chunks of 128 that every unit of a launch runs: at least the two whose
+// DMAs a unit's prologue issues.
+uint32_t k_pairs(int64_t k_slice) { return static_cast<uint32_t>(std::max<int64_t>((k_slice + 127) / 128, 2)); }
+
 // Ungrouped launches pass a NoTaskTable and ntasks = 1; grouped ones the
 // task table and its task count (at most kMaxGroupTasks). `k_slice` is the
 // K of one slice when args.slices > 1.
@@ -739,9 +787,9 @@ hipError_t launch_gemm_cfg(const GemmArgs& args, int64_t k_slice, const PlaneCon
     map.tiles_m = tiles_m;
     map.tiles = make_div_u31(tiles_m * tiles_n);
     map.planes = make_div_u31(args.nplanes);
-    map.group = make_div_u31(static_cast<uint32_t>(kGroupM) * tiles_n);
-    map.rows = make_div_u31(kGroupM);
-    map.tail = make_div_u31(tiles_m - (tiles_m - 1) / kGroupM * kGroupM);
+    map.group = make_div_u31(static_cast<uint32_t>(Cf::kGroupM) * tiles_n);
+    map.rows = make_div_u31(Cf::kGroupM);
+    map.tail = make_div_u31(tiles_m - (tiles_m - 1) / Cf::kGroupM * Cf::kGroupM);
     map.k_begin = static_cast<uint32_t>(kb);
     map.k_stop = static_cast<uint32_t>(kstop);
     map.k_slice = static_cast<uint32_t>(ks);
@@ -749,15 +797,9 @@ hipError_t launch_gemm_cfg(const GemmArgs& args, int64_t k_slice, const PlaneCon
     // share per XCD) when there are at least 8 units
     uint64_t grid = units < slots ? units : slots;
     if (grid >= 8) grid -= grid % 8;
-    // every unit has the same K tiles when the slices divide the range evenly
-    const bool uniform = (kstop - kb) % ks == 0;
-    if (uniform)
-      hipLaunchKernelGGL((plane_gemm_kernel<Cf, kMinBlocks, true, false, kGrouped>), dim3(static_cast<unsigned>(grid)),
-                         dim3(kThreads), 0, stream, args, consts, map, accumulate, tab);
-    else
-      hipLaunchKernelGGL((plane_gemm_kernel<Cf, kMinBlocks, false, false, kGrouped>),
-                         dim3(static_cast<unsigned>(grid)), dim3(kThreads), 0, stream, args, consts, map, accumulate,
-                         tab);
+    map.pairs = k_pairs(ks);
+    hipLaunchKernelGGL((plane_gemm_kernel<Cf, kMinBlocks, false, kGrouped>), dim3(static_cast<unsigned>(grid)),
+                       dim3(Cf::kThreads), 0, stream, args, consts, map, accumulate, tab);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
     if (args.slices > 1) {
@@ -777,6 +819,26 @@ hipError_t launch_gemm_cfg(const GemmArgs& args, int64_t k_slice, const PlaneCon
   return hipSuccess;
 }
 
+// The kernel of `shape`'s tile.
+template <bool kGrouped>
+hipError_t launch_tiles(const GemmShape& shape, const GemmArgs& args, const PlaneConsts& consts, hipStream_t stream,
+                        const GroupArg<kGrouped>& tab, uint32_t ntasks) {
+  switch (shape.tile) {
+    case GemmTile::k256x256:
+      return launch_gemm_cfg<Cfg256x256, 1, kGrouped>(args, shape.k_slice, consts, stream, tab, ntasks);
+    case GemmTile::k256x128:
+      return launch_gemm_cfg<Cfg256x128, 1, kGrouped>(args, shape.k_slice, consts, stream, tab, ntasks);
+    case GemmTile::k128x256:
+      return launch_gemm_cfg<Cfg128x256, 1, kGrouped>(args, shape.k_slice, consts, stream, tab, ntasks);
+    case GemmTile::k128x128:
+      return launch_gemm_cfg<Cfg128x128, 2, kGrouped>(args, shape.k_slice, consts, stream, tab, ntasks);
+    case GemmTile::k64x64:
+      return launch_gemm_cfg<Cfg64x64, 4, kGrouped>(args, shape.k_slice, consts, stream, tab, ntasks);
+    default:
+      return hipErrorInvalidValue;
+  }
+}
+
 }  // namespace
 
 namespace {
@@ -794,9 +856,10 @@ hipError_t launch_listed(const GemmArgs& args, const PlaneConsts& consts, const 
     map.k_begin = static_cast<uint32_t>(kb);
     map.k_stop = static_cast<uint32_t>(kstop);
     map.k_slice = static_cast<uint32_t>(kstop - kb);
+    map.pairs = k_pairs(kstop - kb);
     map.list = d_units;
-    hipLaunchKernelGGL((plane_gemm_kernel<Cf, kMinBlocks, true, true>), dim3(static_cast<unsigned>(grid)),
-                       dim3(kThreads), 0, stream, args, consts, map, kb > 0 ? 1u : 0u, NoTaskTable{});
+    hipLaunchKernelGGL((plane_gemm_kernel<Cf, kMinBlocks, true>), dim3(static_cast<unsigned>(grid)),
+                       dim3(Cf::kThreads), 0, stream, args, consts, map, kb > 0 ? 1u : 0u, NoTaskTable{});
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
   }
@@ -810,8 +873,8 @@ hipError_t launch_gemm_listed(const GemmArgs& args, const PlaneConsts& consts, c
   // the list's entries are checked against the shape and edge where it is built
   if (!gemm_args_ok(args) || args.slices != 1 || !d_units || units > 0x7FFFFFFFu) return hipErrorInvalidValue;
   if (units == 0) return hipSuccess;
-  if (edge == 256) return launch_listed<CfgLarge, 1>(args, consts, d_units, units, stream);
-  if (edge == 128) return launch_listed<CfgSmall, 2>(args, consts, d_units, units, stream);
+  if (edge == 256) return launch_listed<Cfg256x256, 1>(args, consts, d_units, units, stream);
+  if (edge == 128) return launch_listed<Cfg128x128, 2>(args, consts, d_units, units, stream);
   return hipErrorInvalidValue;
 }
 
@@ -864,15 +927,14 @@ hipError_t launch_gemm(const GemmArgs& args, const PlaneConsts& consts, hipStrea
   // split (an unsplit call of a split shape runs unsplit where the kernel
   // allows it)
   if (args.slices > 1 && args.slices != shape.slices) return hipErrorInvalidValue;
-  if (shape.tile == 16) {
+  if (shape.tile == GemmTile::kSkinny) {
     if (args.slices == shape.slices) return launch_skinny(args, shape, consts, stream);
     // an unsplit call (no workspace) of a shape the skinny kernel would
     // split: the 128 x 128 kernel, which takes any K in 65536 blocks
     if (args.slices != 1) return hipErrorInvalidValue;
-    return launch_gemm_cfg<CfgSmall, 2, false>(args, args.k, consts, stream, NoTaskTable{}, 1);
+    return launch_gemm_cfg<Cfg128x128, 2, false>(args, args.k, consts, stream, NoTaskTable{}, 1);
   }
-  if (shape.tile == 256) return launch_gemm_cfg<CfgLarge, 1, false>(args, shape.k_slice, consts, stream, NoTaskTable{}, 1);
-  return launch_gemm_cfg<CfgSmall, 2, false>(args, shape.k_slice, consts, stream, NoTaskTable{}, 1);
+  return launch_tiles<false>(shape, args, consts, stream, NoTaskTable{}, 1);
 }
 
 hipError_t launch_gemm_grouped(const GemmArgs& shape, const PlaneConsts& consts, const TaskPtrs* tasks,
@@ -889,10 +951,10 @@ hipError_t launch_gemm_grouped(const GemmArgs& shape, const PlaneConsts& consts,
     a.b = tasks[t].b;
     a.c = tasks[t].c;
     a.splitk_ws = tasks[t].ws;
-    a.slices = g.tile == 16 ? shape.slices : g.slices;
+    a.slices = g.tile == GemmTile::kSkinny ? shape.slices : g.slices;
     if (!gemm_args_ok(a)) return hipErrorInvalidValue;
   }
-  if (g.tile == 16) {
+  if (g.tile == GemmTile::kSkinny) {
     // the skinny kernel fills the chip from one task's rows and K slices:
     // one launch per task, each with its own workspace
     for (uint32_t t = 0; t < count; ++t) {
@@ -915,8 +977,7 @@ hipError_t launch_gemm_grouped(const GemmArgs& shape, const PlaneConsts& consts,
     a.c = nullptr;
     a.splitk_ws = nullptr;
     a.slices = g.slices;
-    const hipError_t err = g.tile == 256 ? launch_gemm_cfg<CfgLarge, 1, true>(a, g.k_slice, consts, stream, tab, n)
-                                         : launch_gemm_cfg<CfgSmall, 2, true>(a, g.k_slice, consts, stream, tab, n);
+    const hipError_t err = launch_tiles<true>(g, a, consts, stream, tab, n);
     if (err != hipSuccess) return err;
   }
   return hipSuccess;

@@ -81,23 +81,28 @@ __device__ __forceinline__ uint32_t centered_residue_i32(uint32_t u, const Modul
                        k.m_comp);
 }
 
-// Reads accumulator elements 4g .. 4g+3 of a 32x32 MFMA tile straight from
+// The same for a GEMM accumulator u = sum + kGemmAccBias.
+__device__ __forceinline__ CenteredI32 centered_acc_consts(const ModulusConsts& mc) {
+  return CenteredI32{mc.off_acc - mc.half, in_vgpr(mc.half << mc.q_shift), 256u - mc.m};
+}
+
+// Reads the four accumulator elements of a 16x16 MFMA tile straight from
 // their AGPRs. The asm keeps the accumulators in AGPRs through an epilogue
 // (the compiler otherwise copies all of them to VGPRs at once) and, being
 // volatile, keeps the reads in program order with the epilogue's stores, so
 // only a few values are live at a time; four per statement leave the
 // scheduler four independent chains to interleave.
-typedef int v16i __attribute__((ext_vector_type(16)));
+typedef int v4i_acc __attribute__((ext_vector_type(4)));
 struct Acc4 {
   uint32_t v[4];
 };
-__device__ __forceinline__ Acc4 acc_read4(const v16i& acc, int g) {
+__device__ __forceinline__ Acc4 acc_read4(const v4i_acc& acc) {
   Acc4 r;
   asm volatile(
       "v_accvgpr_read_b32 %0, %4\n\tv_accvgpr_read_b32 %1, %5\n\t"
       "v_accvgpr_read_b32 %2, %6\n\tv_accvgpr_read_b32 %3, %7"
       : "=v"(r.v[0]), "=v"(r.v[1]), "=v"(r.v[2]), "=v"(r.v[3])
-      : "a"(acc[4 * g]), "a"(acc[4 * g + 1]), "a"(acc[4 * g + 2]), "a"(acc[4 * g + 3]));
+      : "a"(acc[0]), "a"(acc[1]), "a"(acc[2]), "a"(acc[3]));
   return r;
 }
 

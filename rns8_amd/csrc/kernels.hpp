@@ -156,8 +156,9 @@ hipError_t launch_gemm_grouped(const GemmArgs& shape, const PlaneConsts& consts,
 // the K split. A split covers the whole K in slices of at most 65536, each
 // writing its centered residues to the int8 workspace, and a finalize adds
 // them; unsplit products with K beyond 65536 run as accumulating launches.
+enum class GemmTile : uint32_t { k256x256, k256x128, k128x256, k128x128, k64x64, kSkinny };
 struct GemmShape {
-  int tile;           // 256, 128, or 16 (skinny kernel)
+  GemmTile tile;
   uint32_t slices;    // K slices (1 = no split)
   int64_t k_slice;    // K of one slice
   uint64_t ws_bytes;  // workspace: slices * nplanes * m * padded_ld(n) bytes when split, else 0

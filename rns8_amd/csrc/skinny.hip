@@ -232,7 +232,7 @@ bool skinny_shape(int64_t m, int64_t n, int64_t k, uint32_t nplanes, GemmShape& 
   if (slices > 1) k_slice = (k_slice + kStepK - 1) / kStepK * kStepK;
   slices = (k + k_slice - 1) / k_slice;
   if (waves * slices > 0x7FFFFFFF) return false;
-  out.tile = 16;
+  out.tile = GemmTile::kSkinny;
   out.slices = static_cast<uint32_t>(slices);
   out.k_slice = k_slice;
   out.ws_bytes = slices > 1 ? static_cast<uint64_t>(slices) * nplanes * static_cast<uint64_t>(m) * 16u : 0u;
@@ -241,7 +241,7 @@ bool skinny_shape(int64_t m, int64_t n, int64_t k, uint32_t nplanes, GemmShape& 
 
 hipError_t launch_skinny(const GemmArgs& g, const GemmShape& shape, const PlaneConsts& consts, hipStream_t stream) {
   // shape limits: 16-byte B and C rows, 32-bit offsets inside a row panel
-  if (g.ldb != 16 || g.ldc != 16 || shape.tile != 16 || g.lda >= (int64_t{1} << 23) || g.k >= (int64_t{1} << 31))
+  if (g.ldb != 16 || g.ldc != 16 || shape.tile != GemmTile::kSkinny || g.lda >= (int64_t{1} << 23) || g.k >= (int64_t{1} << 31))
     return hipErrorInvalidValue;
   if (shape.slices > 1 && !g.splitk_ws) return hipErrorInvalidValue;
   const int rb = rows_per_wave_blocks(g.m);

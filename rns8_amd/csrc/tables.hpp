@@ -31,6 +31,11 @@ constexpr int64_t kSafeKBlock = 65536;
 // Centering: with H = floor(m/2), centered(x) = ((x + H) mod m) - H equals the
 // reference rule "r >= (m+1)/2 ? r - m : r" (cpu_reference.cpp:26-32) for
 // every m >= 2. H is folded into the additive offsets below.
+// Start value of the plane GEMM's accumulators: a GEMM sum is at most 2^30 in
+// magnitude (65536 products of 2^14) plus a carried residue, so sum + bias
+// stays inside [0, 2^32); 0x40800000 is the bit pattern of 4.0f, which an MFMA
+// takes as an inline C operand, and 0 modulo 256.
+constexpr uint32_t kGemmAccBias = 0x40800000u;
 struct ModulusConsts {
   uint32_t m;
   uint32_t half;    // H = floor(m/2)
@@ -40,8 +45,10 @@ struct ModulusConsts {
   uint32_t off_i64; // H + (-2^63 mod m): int64 x read as u = x ^ 2^63
   uint32_t off_u64; // H
   uint32_t off_i32; // H + (-2^31 mod m): int32 acc read as u = acc + 2^31
+  uint32_t off_acc; // H + (-kGemmAccBias mod m): GEMM sums read as u = sum + kGemmAccBias
   // Full-rate quotient for the int32 reduction: s = dot(bytes(u), pow_lo) +
-  // off_i32 never exceeds s_max = 255 * (sum of pow_lo bytes) + off_i32, and
+  // off (off_i32 or off_acc) never exceeds s_max = 255 * (sum of pow_lo bytes)
+  // + max(off_i32, off_acc), and
   // floor(s / m) = mulhi_u24(s << q_shift, q_recip) (make_quot24).
   uint32_t q_shift;
   uint32_t q_recip;
@@ -114,9 +121,10 @@ inline ModulusConsts make_modulus_consts(uint32_t m) {
   c.off_i64 = c.half + static_cast<uint32_t>((m - two63_mod) % m);
   c.off_u64 = c.half;
   c.off_i32 = c.half + static_cast<uint32_t>((m - two31_mod) % m);
+  c.off_acc = c.half + (m - kGemmAccBias % m) % m;
   uint32_t byte_sum = 0;
   for (uint32_t b = 0; b < 4; ++b) byte_sum += (lo >> (8u * b)) & 0xFFu;
-  const Quot24 q = make_quot24(m, 255u * byte_sum + c.off_i32);
+  const Quot24 q = make_quot24(m, 255u * byte_sum + (c.off_i32 > c.off_acc ? c.off_i32 : c.off_acc));
   c.q_shift = q.shift;
   c.q_recip = q.recip;
   uint32_t hi_sum = 0;

@@ -2,9 +2,10 @@
 // sustains on this workload's operand statistics, for the roofline context
 // bench.py reports next to its measured GEMM.
 //
-// One 256-thread workgroup per CU; each wave keeps 16 independent 32x32
-// accumulators and issues v_mfma_i32_32x32x32_i8 back to back from register
-// operands, alternating between two operand sets. With `random` the operand
+// One 256-thread workgroup per CU; each wave keeps 64 independent 16x16
+// accumulators and issues v_mfma_i32_16x16x64_i8 (the plane GEMM's
+// instruction; 32x32x32 sustains 17% less with random operands) back to back
+// from register operands. With `random` the operand
 // bytes are a hash of the lane and register index (uniform bytes, like the
 // centered residue planes); otherwise they are zero. Each workgroup records
 // its elapsed shader cycles (s_memtime) and 100 MHz reference ticks
@@ -17,7 +18,6 @@
 namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v16i __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ uint32_t mix(uint32_t x) {
   x ^= x >> 16;
@@ -30,42 +30,36 @@ __device__ __forceinline__ uint32_t mix(uint32_t x) {
 __global__ __launch_bounds__(256, 1) void mfma_rate_kernel(int iters, uint32_t random, int* sink,
                                                            unsigned long long* ticks) {
   const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-  v4i a0[4], b0[4], a1[4], b1[4];
+  v4i a[8], b[8];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 8; ++i)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const uint32_t s = g * 64u + 16u * i + e;
-      a0[i][e] = random ? static_cast<int>(mix(s)) : 0;
-      b0[i][e] = random ? static_cast<int>(mix(s + 4u)) : 0;
-      a1[i][e] = random ? static_cast<int>(mix(s + 8u)) : 0;
-      b1[i][e] = random ? static_cast<int>(mix(s + 12u)) : 0;
+      const uint32_t s = g * 64u + 4u * i + e;
+      a[i][e] = random ? static_cast<int>(mix(s)) : 0;
+      b[i][e] = random ? static_cast<int>(mix(s + 32u)) : 0;
     }
-  v16i acc[4][4];
+  v4i acc[8][8];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 8; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = v16i{};
+    for (int j = 0; j < 8; ++j) acc[i][j] = v4i{};
   __syncthreads();
   const unsigned long long c0 = __builtin_readcyclecounter();
   const unsigned long long r0 = __builtin_amdgcn_s_memrealtime();
   for (int it = 0; it < iters; ++it) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 8; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(b0[j], a0[i], acc[i][j], 0, 0, 0);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(b1[j], a1[i], acc[i][j], 0, 0, 0);
+      for (int j = 0; j < 8; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(b[j], a[i], acc[i][j], 0, 0, 0);
   }
   const unsigned long long c1 = __builtin_readcyclecounter();
   const unsigned long long r1 = __builtin_amdgcn_s_memrealtime();
   int s = 0;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 8; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) s ^= acc[i][j][0] ^ acc[i][j][15];
+    for (int j = 0; j < 8; ++j) s ^= acc[i][j][0] ^ acc[i][j][3];
   sink[g] = s;
   if (threadIdx.x == 0) {
     ticks[2 * blockIdx.x] = c1 - c0;
@@ -121,7 +115,7 @@ extern "C" __attribute__((visibility("default"))) int rns8_probe_mfma_rate(int r
       ghz += static_cast<double>(h[2 * b]) / (static_cast<double>(h[2 * b + 1]) * 10.0);  // 100 MHz ticks
       ++n;
     }
-  const double ops = static_cast<double>(cus) * 4.0 * iters * 32.0 * 65536.0 * launches;
+  const double ops = static_cast<double>(cus) * 4.0 * iters * 64.0 * 32768.0 * launches;
   *tops = ms > 0.f ? ops / (ms * 1e-3) / 1e12 : 0.0;
   *clock_ghz = n ? ghz / n : 0.0;
   return done(hipSuccess);
