@@ -100,7 +100,7 @@ rns8_status pack_native(rns8_context* ctx, rns8_matrix* matrix, const T* src, in
     }
   }
   const PackArgs args = pack_args(*matrix, dsrc, dld, is_signed);
-  if (launch_pack_native(args, make_ladder_plane_consts(matrix->prefix), stream) != hipSuccess)
+  if (launch_pack_native(args, stream) != hipSuccess)
     return RNS8_BACKEND_FAILURE;
   if (is_wide) {
     const rns8_status st = commit_native_proof(*matrix, proof_max, pending, stream);

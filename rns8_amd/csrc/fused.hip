@@ -46,6 +46,7 @@
 #include "dma.hpp"
 #include "int_ops.hpp"
 #include "kernels.hpp"
+#include "plane_consts.hpp"
 
 namespace rns8x {
 namespace {
@@ -112,8 +113,8 @@ __global__ __launch_bounds__(kThreads, 1) void fused_native_kernel(FusedArgs a, 
   // padding (strides are even); the epilogue stores zero for that column.
   const bool is_a = wave < 8;
   const int c = wave & 7;
-  const ModulusConsts mc0 = pc.mod[p0];
-  const ModulusConsts mc1 = pc.mod[NP > 1 ? p0 + 1 : p0];
+  const ModulusConsts mc0 = plane_mod(pc, p0);
+  const ModulusConsts mc1 = plane_mod(pc, NP > 1 ? p0 + 1 : p0);
   const int ra = 16 * c + (lane >> 4);                 // an A lane's first row (then +4 per load)
   const int kfirst = is_a ? 2 * (lane & 15) : 4 * c;  // the lane's first k within a step
   const uint32_t lda8 = static_cast<uint32_t>(a.lda) * 8u, ldb8 = static_cast<uint32_t>(a.ldb) * 8u;
@@ -374,7 +375,7 @@ __global__ __launch_bounds__(256) void residue_finalize_kernel(const int8_t* ws,
         for (int e = 0; e < 16; ++e) sum[e] += part[g][e][lc];
       const uint32_t plane = static_cast<uint32_t>(ch / chunks_per_plane);
       const int64_t in_plane = ch - static_cast<int64_t>(plane) * chunks_per_plane;
-      const ModulusConsts mc = pc.mod[plane];
+      const ModulusConsts mc = plane_mod(pc, plane);
       const CenteredI32 kc = centered_i32_consts(mc);
       v4i out;
 #pragma unroll

@@ -54,6 +54,7 @@
 #include "dma.hpp"
 #include "int_ops.hpp"
 #include "kernels.hpp"
+#include "plane_consts.hpp"
 
 namespace rns8x {
 namespace {
@@ -118,7 +119,7 @@ __global__ __launch_bounds__(256) void pack_bt_kernel(const uint64_t* b, int64_t
       hi[e] = static_cast<uint32_t>(x >> 32);
     }
     const uint32_t p = blockIdx.y;
-    const ModulusConsts mc = pc.mod[p];
+    const ModulusConsts mc = plane_mod(pc, p);
     uint32_t r[16];
 #pragma unroll
     for (int e = 0; e < 16; ++e) r[e] = residue64<Signed>(lo[e], hi[e], mc);
@@ -258,9 +259,9 @@ __global__ __launch_bounds__(kThreads, kMinBlocks) void fused_skinny_kernel(Skin
 #pragma unroll
       for (int p = 0; p < G; ++p) {
         if (kFirst256 && p == 0)
-          plane_mma(fast, std::true_type{}, lo, hi, stage, p, acc[p], pc.mod[0]);
+          plane_mma(fast, std::true_type{}, lo, hi, stage, p, acc[p], plane_mod(pc, 0));
         else
-          plane_mma(fast, std::false_type{}, lo, hi, stage, p, acc[p], pc.mod[p0 + p]);
+          plane_mma(fast, std::false_type{}, lo, hi, stage, p, acc[p], plane_mod(pc, p0 + p));
       }
     };
     auto compute = [&](const Raw& x, int stage) {
@@ -324,7 +325,7 @@ __global__ __launch_bounds__(kThreads, kMinBlocks) void fused_skinny_kernel(Skin
   const uint32_t row = row0 + static_cast<uint32_t>(frow);
 #pragma unroll
   for (int p = 0; p < G; ++p) {
-    const ModulusConsts mc = pc.mod[p0 + p];
+    const ModulusConsts mc = plane_mod(pc, p0 + p);
     const CenteredI32 kc = centered_i32_consts(mc);
     uint32_t r[4];
 #pragma unroll

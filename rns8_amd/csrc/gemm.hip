@@ -63,6 +63,7 @@
 #include "dma.hpp"
 #include "int_ops.hpp"
 #include "kernels.hpp"
+#include "plane_consts.hpp"
 
 namespace rns8x {
 namespace {
@@ -425,7 +426,7 @@ __global__ __launch_bounds__(C::kThreads, kMinBlocks) void plane_gemm_kernel(Gem
     // states after the last MFMA for them: 24 here cover the longest
     // MFMA-write to v_accvgpr_read dependency.
     asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7");
-    const ModulusConsts mc = pc.mod[U.plane];
+    const ModulusConsts mc = plane_mod(pc, U.plane);
     const int64_t tile_rows = min(static_cast<int64_t>(BM), args.m - U.m0);
     const uint32_t lane_off =
         static_cast<uint32_t>((wave_m * (16 * TM) + frag_row) * args.ldc + wave_n * (16 * TN));

@@ -29,7 +29,7 @@ struct PackArgs {
   uint32_t nplanes;
   NativeKind kind;
 };
-hipError_t launch_pack_native(const PackArgs& args, const PlaneConsts& consts, hipStream_t stream);
+hipError_t launch_pack_native(const PackArgs& args, hipStream_t stream);
 
 // ---- exact-wide magnitude proofs (exact_axes.hip) ---------------------------
 // Per-row and per-column summaries of a rows x cols native operand (row

@@ -27,8 +27,7 @@ typedef unsigned long long v2u64 __attribute__((ext_vector_type(2)));
 // matrices with 2^32 chunks or more). With kStream the plane stores are
 // non-temporal (see kStreamPackBytes).
 template <bool Signed, bool Vec, bool kStream>
-__global__ __launch_bounds__(256) void pack_native_kernel(PackArgs a, PlaneConsts pc, uint32_t chunks_per_row,
-                                                          uint32_t total_chunks) {
+__global__ __launch_bounds__(256) void pack_native_kernel(PackArgs a, uint32_t chunks_per_row, uint32_t total_chunks) {
   constexpr int kCols = 8;
   const uint64_t* const src = static_cast<const uint64_t*>(a.src);
   for (uint32_t ch = blockIdx.x * blockDim.x + threadIdx.x; ch < total_chunks; ch += gridDim.x * blockDim.x) {
@@ -55,15 +54,16 @@ __global__ __launch_bounds__(256) void pack_native_kernel(PackArgs a, PlaneConst
       }
     }
     pack_chunk8<Signed, kStream>(lo, hi, a.planes + static_cast<int64_t>(row) * a.plane_ld + c0, a.plane_pitch,
-                                 a.nplanes, pc, true);
+                                 a.nplanes, true);
   }
 }
 
 // Finite u8: x < 256, s = x + H < 2^9 is inside the range of the int32
 // reduction constants (their s_max is at least 255 + H), and x itself is
 // s - H (centered_byte).
-__global__ __launch_bounds__(256) void pack_u8_kernel(PackU8Args a, ModulusConsts mc, uint32_t chunks_per_row,
-                                                      uint32_t total_chunks, uint32_t vec_load) {
+__global__ __launch_bounds__(256) void pack_u8_kernel(PackU8Args a, uint32_t chunks_per_row, uint32_t total_chunks,
+                                                      uint32_t vec_load) {
+  const ModulusConsts& mc = plane_mod(PlaneConsts{a.modulus}, 0);
   const uint32_t m_comp = 256u - mc.m;
   const uint32_t h_sh = in_vgpr(mc.half << mc.q_shift);
   for (uint32_t ch = blockIdx.x * blockDim.x + threadIdx.x; ch < total_chunks; ch += gridDim.x * blockDim.x) {
@@ -107,7 +107,7 @@ unsigned grid_for(int64_t items) {
 
 }  // namespace
 
-hipError_t launch_pack_native(const PackArgs& a, const PlaneConsts& consts, hipStream_t stream) {
+hipError_t launch_pack_native(const PackArgs& a, hipStream_t stream) {
   if (!pack_args_ok(a)) return hipErrorInvalidValue;
   const int64_t chunks_per_row = a.plane_ld / 8;
   const int64_t total = chunks_per_row * a.rows;
@@ -118,7 +118,7 @@ hipError_t launch_pack_native(const PackArgs& a, const PlaneConsts& consts, hipS
                           kStreamPackBytes;
   auto launch_as = [&](auto sgn, auto vc, auto st) {
     hipLaunchKernelGGL((pack_native_kernel<decltype(sgn)::value, decltype(vc)::value, decltype(st)::value>), grid,
-                       dim3(256), 0, stream, a, consts, cpr, tot);
+                       dim3(256), 0, stream, a, cpr, tot);
   };
   using T = std::true_type;
   using F = std::false_type;
@@ -141,7 +141,7 @@ hipError_t launch_pack_u8(const PackU8Args& a, hipStream_t stream) {
   const int64_t chunks_per_row = a.plane_ld / 16;
   const int64_t total = chunks_per_row * a.rows;
   const uint32_t vec = (reinterpret_cast<uintptr_t>(a.src) % 16 == 0 && a.ld % 16 == 0) ? 1u : 0u;
-  hipLaunchKernelGGL(pack_u8_kernel, dim3(grid_for(total)), dim3(256), 0, stream, a, make_modulus_consts(a.modulus),
+  hipLaunchKernelGGL(pack_u8_kernel, dim3(grid_for(total)), dim3(256), 0, stream, a,
                      static_cast<uint32_t>(chunks_per_row), static_cast<uint32_t>(total), vec);
   return hipGetLastError();
 }

@@ -37,6 +37,7 @@
 #include "dma.hpp"
 #include "int_ops.hpp"
 #include "kernels.hpp"
+#include "plane_consts.hpp"
 
 namespace rns8x {
 namespace {
@@ -196,7 +197,7 @@ __global__ __launch_bounds__(kThreads) void skinny_gemm_kernel(SkinnyArgs a, Pla
 
   // Epilogue: lane l holds u = 2^31 + C[row0 + 16 rb + l % 16][4 (l / 16) + e]
   // in element e of acc[rb].
-  const ModulusConsts mc = pc.mod[plane];
+  const ModulusConsts mc = plane_mod(pc, plane);
   const CenteredI32 kc = centered_i32_consts(mc);
   int8_t* const dst = a.dst + (static_cast<uint64_t>(slice) * a.nplanes + plane) * a.pitch_dst;
 #pragma unroll

@@ -100,7 +100,7 @@ constexpr uint32_t div_u31_host(uint32_t n, DivU31 v) {
   return static_cast<uint32_t>((static_cast<uint64_t>(n << 1) * v.mul) >> 32) >> v.shift;
 }
 
-inline ModulusConsts make_modulus_consts(uint32_t m) {
+constexpr ModulusConsts make_modulus_consts(uint32_t m) {
   ModulusConsts c{};
   c.m = m;
   c.half = m / 2u;
@@ -136,21 +136,29 @@ inline ModulusConsts make_modulus_consts(uint32_t m) {
   return c;
 }
 
-// Up to kMaxPrefix planes of modulus constants, passed by value to kernels.
+// Which moduli a launch's planes have: the ladder's first planes, or one plane
+// of a finite modulus. Kernels take this and read their constants from a table
+// in device memory (plane_consts.hpp).
 struct PlaneConsts {
-  ModulusConsts mod[kMaxPrefix];
+  uint32_t modulus;  // 0: plane p has modulus kLadder[p]
 };
 
-inline PlaneConsts make_ladder_plane_consts(uint32_t prefix) {
-  PlaneConsts pc{};
-  for (uint32_t p = 0; p < prefix && p < kMaxPrefix; ++p) pc.mod[p] = make_modulus_consts(kLadder[p]);
-  return pc;
-}
+inline PlaneConsts make_ladder_plane_consts(uint32_t) { return PlaneConsts{0}; }
+inline PlaneConsts make_single_plane_consts(uint32_t modulus) { return PlaneConsts{modulus}; }
 
-inline PlaneConsts make_single_plane_consts(uint32_t modulus) {
-  PlaneConsts pc{};
-  pc.mod[0] = make_modulus_consts(modulus);
-  return pc;
+// The table: the ladder's kMaxPrefix moduli, then every modulus 0 .. 256 (0
+// and 1 unused).
+struct ModulusTable {
+  ModulusConsts entry[kMaxPrefix + 257];
+};
+constexpr ModulusTable make_modulus_table() {
+  ModulusTable t{};
+  for (uint32_t p = 0; p < kMaxPrefix; ++p) t.entry[p] = make_modulus_consts(kLadder[p]);
+  for (uint32_t m = 2; m <= 256; ++m) t.entry[kMaxPrefix + m] = make_modulus_consts(m);
+  return t;
+}
+constexpr uint32_t modulus_table_index(PlaneConsts pc, uint32_t plane) {
+  return pc.modulus ? kMaxPrefix + pc.modulus : plane;
 }
 
 // ---- Garner reconstruction ---------------------------------------------------
