@@ -34,14 +34,15 @@ hipError_t launch_pack_native(const PackArgs& args, hipStream_t stream);
 // ---- exact-wide magnitude proofs (exact_axes.hip) ---------------------------
 // Per-row and per-column summaries of a rows x cols native operand (row
 // stride ld elements) into out_rows / out_cols, and its max |x| into
-// words[0] (words[1..7] zero). row_part / col_part: scratch for
-// native_partial_rows(rows, cols) and native_partial_cols(rows, cols)
-// partials (one per axis and 64 x 64 tile).
+// words[0] (words[1..7] zero). ticket: zero before the matrix's first launch;
+// every launch leaves it zero. Launches on one ticket are ordered.
+struct ProofTicket {
+  unsigned long long best;
+  uint32_t drawn, unused;
+};
 hipError_t launch_native_axes(const void* src, int64_t rows, int64_t cols, int64_t ld, bool is_signed,
-                              xa::AxisPartial* row_part, xa::AxisPartial* col_part, xa::AxisRecord* out_rows,
-                              xa::AxisRecord* out_cols, uint64_t* words, hipStream_t stream);
-inline int64_t native_partial_rows(int64_t rows, int64_t cols) { return rows * ((cols + 63) / 64); }
-inline int64_t native_partial_cols(int64_t rows, int64_t cols) { return cols * ((rows + 63) / 64); }
+                              xa::AxisRecord* out_rows, xa::AxisRecord* out_cols, uint64_t* words,
+                              ProofTicket* ticket, hipStream_t stream);
 // The carried summaries of C = A x B (m x n, inner k): per-row and
 // per-column maxima and sums of the cell bounds from A's m row records and
 // B's n column records (kinds: xa::AxisKind; a uniform side reads no
