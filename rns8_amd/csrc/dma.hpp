@@ -56,7 +56,14 @@ __device__ __forceinline__ void dma16(uint32_t lds_addr, uint32_t voffset, v4i r
                : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voffset), "s"(rsrc)
                : "m0");
 }
-// The same to lds_base + 1024 * block (block a constant below 8 once the
+// The same, non-temporal: for operands read once.
+__device__ __forceinline__ void dma16_stream(uint32_t lds_addr, uint32_t voffset, v4i rsrc) {
+  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds"
+               :
+               : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voffset), "s"(rsrc)
+               : "m0");
+}
+// The same (ordinary) to lds_base + 1024 * block (block a constant below 8 once the
 // caller's loop is unrolled): the offset is the addition's literal, so a block
 // costs one scalar instruction beside its load.
 template <int kBlock>

@@ -5,6 +5,9 @@
 // operands inside its tile loads; its N <= 8 GEMV is
 // hip_direct_gemm_tiled_kernels.cuh:298-432).
 //
+// Products whose planes x columns fill few 16-column groups run in
+// fused_digits.hip instead (fused_digits_shape says which).
+//
 // The packed route writes every residue plane of A to HBM and reads it back:
 // at 8192 x 1 x 8192 with 9 planes that is 537 MB read, 604 MB written and
 // 604 MB read again. Here A's 537 MB are read once and each element is
@@ -379,12 +382,15 @@ bool fused_skinny_shape(int64_t m, int64_t n, int64_t k, uint32_t nplanes, Fused
   out.ws_bytes = bt + slots;
   out.skinny = 1;
   out.bt_bytes = bt;
+  // (which products are accepted stays this form's rule)
+  FusedShape digits;
+  if (fused_digits_shape(m, n, k, nplanes, digits)) out = digits;
   return true;
 }
 
 hipError_t launch_fused_skinny(const FusedArgs& f, const PlaneConsts& consts, hipStream_t stream) {
   const FusedShape& sh = f.shape;
-  if (!sh.skinny || f.ldc != 16 || f.n > 16 || f.k > kMaxK || f.lda >= (int64_t{1} << 21)) return hipErrorInvalidValue;
+  if (sh.skinny != 1 || f.ldc != 16 || f.n > 16 || f.k > kMaxK || f.lda >= (int64_t{1} << 21)) return hipErrorInvalidValue;
   const int64_t kp = kp_of(f.k);
   const bool sgn = f.kind == NativeKind::I64;
   // B's transposed residue planes at the start of the workspace
