@@ -37,7 +37,10 @@
 //
 // Each slice reduces its int32 sums to centered int8 residues in the
 // epilogue and stores them into its own slot of the workspace; a finalize
-// kernel adds the slices' residues and reduces once more. Partial residues
+// kernel adds the slices' residues and reduces once more. An odd last plane is
+// a workgroup of the same grid that converts and multiplies one plane: as a
+// launch of its own behind the pairs it took as long as they do (128 x 128 x
+// 65536, 9 planes: 100 us, now 85; 8 planes 59). Partial residues
 // are a quarter of the bytes of int32 partial sums, and slices of at most
 // 65536 K keep every int32 sum exact.
 #include <algorithm>
@@ -67,6 +70,7 @@ constexpr int kLdsBytes = 2 * kStageLds;             // two stages
 constexpr int64_t kMaxSliceK = 65536;                // |int32 sum| <= 65536 * 128 * 128 = 2^30
 constexpr int64_t kMinSliceK = 512;                  // 16 steps: amortizes the epilogue
 constexpr uint64_t kMaxWorkspace = uint64_t{64} << 20;
+constexpr int64_t kSliceSteps = 6;                   // a slice's start and epilogue, in steps
 constexpr uint32_t kOutOfRange = 0x80000000u;        // a buffer offset past every resource
 
 // A lane's four 16-byte loads of one step, as issued. Element (j, h) is
@@ -77,14 +81,27 @@ struct Raw {
   v4i v[4];
 };
 
+// Reads what the conversion uses of a modulus' record here, into scalar
+// registers the compiler knows to be the wave's: left to their first uses, the
+// reads are sunk into the conversion's branches and the branches on them grow
+// (128 x 128 x 65536, 8 planes: 1.2 us).
+template <bool Signed>
+__device__ __forceinline__ void hold_consts(ModulusConsts& mc) {
+  asm volatile("" : "+s"(mc.m), "+s"(mc.half), "+s"(mc.pow_lo), "+s"(mc.pow_hi), "+s"(mc.pq_shift), "+s"(mc.pq_recip),
+                    "+s"(Signed ? mc.off_i64 : mc.off_u64));
+  if constexpr (Signed) asm volatile("" : "+s"(mc.off_i32), "+s"(mc.q_shift), "+s"(mc.q_recip));
+}
+
 // Grid: x = output tile (tiles_n per tile row), y = K slice, z = plane pair
-// (planes p0 .. p0 + NP - 1, p0 = plane_base + 2 * z). The host guarantees
+// (planes 2 z and 2 z + 1; of an odd count the last pair has one). The host guarantees
 // every slice holds at least one K element, 16-byte aligned operands with
 // even row strides, and row strides below 2^21 elements.
-template <bool Signed, int NP>
-__global__ __launch_bounds__(kThreads, 1) void fused_native_kernel(FusedArgs a, PlaneConsts pc, uint32_t tiles_n,
-                                                                   uint32_t plane_base) {
+template <bool Signed>
+__global__ __launch_bounds__(kThreads, 1) void fused_native_kernel(FusedArgs a, PlaneConsts pc, uint32_t tiles_n) {
   __shared__ __attribute__((aligned(16))) int8_t lds[kLdsBytes];
+  // every argument line is requested before the first wait
+  asm volatile("" ::"s"(a.a), "s"(a.b), "s"(a.lda), "s"(a.ldb), "s"(a.m), "s"(a.n), "s"(a.k), "s"(a.shape.k_slice),
+               "s"(a.nplanes), "s"(pc.modulus), "s"(tiles_n));
   const int t = threadIdx.x;
   const int lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -93,7 +110,8 @@ __global__ __launch_bounds__(kThreads, 1) void fused_native_kernel(FusedArgs a, 
   const int64_t m0 = static_cast<int64_t>(tr) * kTileM;
   const int64_t n0 = static_cast<int64_t>(tc) * kTileN;
   const uint32_t slice = blockIdx.y;
-  const uint32_t p0 = plane_base + blockIdx.z * kGroupPlanes;
+  const uint32_t p0 = blockIdx.z * kGroupPlanes;
+  const bool two = p0 + 1 < a.nplanes;
   const int64_t kb = static_cast<int64_t>(slice) * a.shape.k_slice;
   const int64_t ke = min(kb + a.shape.k_slice, a.k);
   const int steps = static_cast<int>((ke - kb + kStepK - 1) / kStepK);
@@ -113,8 +131,7 @@ __global__ __launch_bounds__(kThreads, 1) void fused_native_kernel(FusedArgs a, 
   // padding (strides are even); the epilogue stores zero for that column.
   const bool is_a = wave < 8;
   const int c = wave & 7;
-  const ModulusConsts mc0 = plane_mod(pc, p0);
-  const ModulusConsts mc1 = plane_mod(pc, NP > 1 ? p0 + 1 : p0);
+  ModulusConsts mc0, mc1;  // read below, behind the first operand loads
   const int ra = 16 * c + (lane >> 4);                 // an A lane's first row (then +4 per load)
   const int kfirst = is_a ? 2 * (lane & 15) : 4 * c;  // the lane's first k within a step
   const uint32_t lda8 = static_cast<uint32_t>(a.lda) * 8u, ldb8 = static_cast<uint32_t>(a.ldb) * 8u;
@@ -247,10 +264,10 @@ __global__ __launch_bounds__(kThreads, 1) void fused_native_kernel(FusedArgs a, 
     // one branch per wave: the 32-bit form when no lane has a wide element
     if (__builtin_amdgcn_ballot_w64(wide != 0u) == 0u) {
       plane_of(std::true_type{}, x, mc0, off);
-      if constexpr (NP > 1) plane_of(std::true_type{}, x, mc1, off + kPlaneLds);
+      if (two) plane_of(std::true_type{}, x, mc1, off + kPlaneLds);
     } else {
       plane_of(std::false_type{}, x, mc0, off);
-      if constexpr (NP > 1) plane_of(std::false_type{}, x, mc1, off + kPlaneLds);
+      if (two) plane_of(std::false_type{}, x, mc1, off + kPlaneLds);
     }
   };
 
@@ -262,7 +279,7 @@ __global__ __launch_bounds__(kThreads, 1) void fused_native_kernel(FusedArgs a, 
   // C[row][col] with row = m0 + 64 wm + 32 i + (l & 31) and col = n0 + 64 wn +
   // 32 hn + 8 g + 4 (l >> 5) + e.
   const int pl = wave >> 3, wm = (wave >> 2) & 1, wn = (wave >> 1) & 1, hn = wave & 1;
-  const bool mfma_wave = pl < NP;
+  const bool mfma_wave = pl == 0 || two;
   const int frag = (lane >> 5) * kChunkLds + (lane & 31) * 16;
   v16i acc[2] = {v16i{}, v16i{}};
   auto mma = [&](int stage) {
@@ -295,6 +312,13 @@ __global__ __launch_bounds__(kThreads, 1) void fused_native_kernel(FusedArgs a, 
   };
   Raw r0, r1;
   load(r0, 0);
+  // both planes' constants at once, while the first values are in flight
+  uint32_t first_plane = p0;
+  asm volatile("" : "+s"(first_plane)::"memory");
+  mc0 = plane_mod(pc, first_plane);
+  mc1 = plane_mod(pc, two ? first_plane + 1 : first_plane);
+  hold_consts<Signed>(mc0);
+  hold_consts<Signed>(mc1);
   for (int s = 0;;) {
     step(r0, r1, s);
     if (++s >= steps) break;
@@ -409,17 +433,30 @@ bool choose_fused_shape(int64_t m, int64_t n, int64_t k, uint32_t nplanes, int64
   const int64_t tiles = ((m + kTileM - 1) / kTileM) * ((n + kTileN - 1) / kTileN);
   const int64_t groups = (nplanes + kGroupPlanes - 1) / kGroupPlanes;
   if (tiles >= (int64_t{1} << 31)) return false;
-  // about one workgroup per CU, slices of at least kMinSliceK and at most
-  // kMaxSliceK, every slice non-empty
-  const int64_t target = (256 + tiles * groups - 1) / (tiles * groups);
-  int64_t slices = std::max((k + kMaxSliceK - 1) / kMaxSliceK, std::min(target, (k + kMinSliceK - 1) / kMinSliceK));
-  slices = std::max<int64_t>(slices, 1);
-  int64_t k_slice = (k + slices - 1) / slices;
-  k_slice = (k_slice + kStepK - 1) / kStepK * kStepK;
-  slices = (k + k_slice - 1) / k_slice;
-  if (slices > 65535) return false;
-  const uint64_t bytes = static_cast<uint64_t>(slices) * nplanes * static_cast<uint64_t>(m) * static_cast<uint64_t>(ldc);
-  if (bytes > kMaxWorkspace) return false;
+  const int64_t work = tiles * groups;  // workgroups per slice
+  const int64_t least = std::max<int64_t>((k + kMaxSliceK - 1) / kMaxSliceK, 1);
+  auto fit = [&](int64_t want, int64_t& slices, int64_t& k_slice, uint64_t& bytes) {
+    slices = std::max(least, std::min(want, (k + kMinSliceK - 1) / kMinSliceK));
+    k_slice = ((k + slices - 1) / slices + kStepK - 1) / kStepK * kStepK;
+    slices = (k + k_slice - 1) / k_slice;  // every slice holds at least one k
+    bytes = static_cast<uint64_t>(slices) * nplanes * static_cast<uint64_t>(m) * static_cast<uint64_t>(ldc);
+    return slices <= 65535 && bytes <= kMaxWorkspace;
+  };
+  // The path is offered when slices for at least one workgroup per CU fit the
+  // workspace. Of those and the slices that fill one to three rounds of CUs
+  // (one workgroup each), the least rounds x steps of a slice runs, a slice's
+  // start and epilogue counted as kSliceSteps steps: 258 workgroups take two
+  // rounds where 252 take one (64 x 200 x 30000, 5 planes: 56 against 44 us;
+  // 200 x 200 x 4000, 5 planes 44 against 30).
+  int64_t slices, k_slice;
+  uint64_t bytes;
+  if (!fit((256 + work - 1) / work, slices, k_slice, bytes)) return false;
+  auto cost = [&](int64_t sl, int64_t ks) { return (work * sl + 255) / 256 * (ks / kStepK + kSliceSteps); };
+  for (int64_t rounds = 1; rounds <= 3; ++rounds) {
+    int64_t sl, ks;
+    uint64_t by;
+    if (fit(256 * rounds / work, sl, ks, by) && cost(sl, ks) < cost(slices, k_slice)) slices = sl, k_slice = ks, bytes = by;
+  }
   out.slices = static_cast<uint32_t>(slices);
   out.k_slice = k_slice;
   out.ws_bytes = bytes;
@@ -447,19 +484,11 @@ hipError_t launch_fused_native(const FusedArgs& a, const PlaneConsts& consts, hi
   const uint32_t tiles_n = static_cast<uint32_t>((a.n + kTileN - 1) / kTileN);
   const uint32_t tiles = static_cast<uint32_t>((a.m + kTileM - 1) / kTileM) * tiles_n;
   const bool sgn = a.kind == NativeKind::I64;
-  // full pairs of planes in one grid, an odd last plane in another
-  const uint32_t full = a.nplanes / kGroupPlanes;
-  const uint32_t rest = a.nplanes - full * kGroupPlanes;
-  auto launch = [&](auto np, uint32_t groups, uint32_t base) {
-    constexpr int NP = decltype(np)::value;
-    const dim3 grid(tiles, a.shape.slices, groups);
-    if (sgn)
-      hipLaunchKernelGGL((fused_native_kernel<true, NP>), grid, dim3(kThreads), 0, stream, a, consts, tiles_n, base);
-    else
-      hipLaunchKernelGGL((fused_native_kernel<false, NP>), grid, dim3(kThreads), 0, stream, a, consts, tiles_n, base);
-  };
-  if (full) launch(std::integral_constant<int, kGroupPlanes>{}, full, 0);
-  if (rest) launch(std::integral_constant<int, 1>{}, 1, full * kGroupPlanes);
+  const dim3 grid(tiles, a.shape.slices, (a.nplanes + kGroupPlanes - 1) / kGroupPlanes);
+  if (sgn)
+    hipLaunchKernelGGL(fused_native_kernel<true>, grid, dim3(kThreads), 0, stream, a, consts, tiles_n);
+  else
+    hipLaunchKernelGGL(fused_native_kernel<false>, grid, dim3(kThreads), 0, stream, a, consts, tiles_n);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   return launch_residue_finalize(a.ws, a.c, a.m, a.ldc, a.pitch_c, a.nplanes, a.shape.slices, consts, stream);
