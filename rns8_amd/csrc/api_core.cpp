@@ -1122,7 +1122,6 @@ rns8_status rns8_destroy_matrix(rns8_matrix* matrix) {
     free_device(matrix->planes);
     free_device(matrix->upload);
     free_device(matrix->staging);
-    free_device(matrix->status);
     free_device(matrix->proof_device);
     if (matrix->proof_event) (void)hipEventDestroy(matrix->proof_event);
     delete matrix;

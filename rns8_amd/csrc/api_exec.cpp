@@ -47,7 +47,9 @@ rns8_status sync(hipStream_t s) { return hipStreamSynchronize(s) == hipSuccess ?
 
 // ---- pack ------------------------------------------------------------------------
 
-enum class Source { Host, Device };
+// HostQueued: a host array whose upload and pack are left enqueued on the
+// context's stream (the oneshot calls, which wait once at their end).
+enum class Source { Host, HostQueued, Device };
 
 template <typename T>
 rns8_status pack_native(rns8_context* ctx, rns8_matrix* matrix, const T* src, int64_t ld, uint64_t sv, Source where,
@@ -74,7 +76,7 @@ rns8_status pack_native(rns8_context* ctx, rns8_matrix* matrix, const T* src, in
   if (same_source) return RNS8_SUCCESS;
   const void* dsrc = src;
   int64_t dld = ld;
-  if (where == Source::Host) {
+  if (where != Source::Device) {
     const std::size_t bytes = static_cast<std::size_t>(rows) * cols * sizeof(T);
     rns8_status st = ensure_device_buffer(ctx->device_id, &matrix->upload, &matrix->upload_bytes, bytes);
     if (st != RNS8_SUCCESS) return st;
@@ -128,7 +130,7 @@ rns8_status pack_u8(rns8_context* ctx, rns8_matrix* matrix, uint16_t modulus, co
   if (hipSetDevice(ctx->device_id) != hipSuccess) return RNS8_BACKEND_FAILURE;
   const uint8_t* dsrc = src;
   int64_t dld = ld;
-  if (where == Source::Host) {
+  if (where != Source::Device) {
     const std::size_t bytes = static_cast<std::size_t>(rows) * cols;
     rns8_status st = ensure_device_buffer(ctx->device_id, &matrix->upload, &matrix->upload_bytes, bytes);
     if (st != RNS8_SUCCESS) return st;
@@ -435,20 +437,18 @@ rns8_status export_host(rns8_context* ctx, const rns8_plan* plan, const rns8_mat
   const std::size_t elem = sizeof(uint64_t) * req.limbs;
   const std::size_t bytes = static_cast<std::size_t>(m) * n * elem;
   if (hipSetDevice(ctx->device_id) != hipSuccess) return RNS8_BACKEND_FAILURE;
-  st = ensure_device_buffer(ctx->device_id, &mc->staging, &mc->staging_bytes, bytes);
+  // the status word lies right behind the cells, so both come in one transfer
+  st = ensure_device_buffer(ctx->device_id, &mc->staging, &mc->staging_bytes, bytes + sizeof(uint64_t));
   if (st != RNS8_SUCCESS) return st;
-  if (!mc->status && hipMalloc(reinterpret_cast<void**>(&mc->status), 64) != hipSuccess) return RNS8_BACKEND_FAILURE;
+  auto* const d_status = reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(mc->staging) + bytes);
   const hipStream_t stream = ctx->stream;
-  if (launch_zero_words(mc->status, 1, stream) != hipSuccess) return RNS8_BACKEND_FAILURE;
-  const ExportArgs a = export_args(*plan, *C, mc->staging, n, req.limbs, req.kind, mc->status);
+  if (launch_zero_words(d_status, 1, stream) != hipSuccess) return RNS8_BACKEND_FAILURE;
+  const ExportArgs a = export_args(*plan, *C, mc->staging, n, req.limbs, req.kind, d_status);
   if (launch_plan_export(*plan, a, stream) != hipSuccess) return RNS8_BACKEND_FAILURE;
   uint32_t status = 0;
-  if (hipMemcpyAsync(&status, mc->status, sizeof(status), hipMemcpyDeviceToHost, stream) != hipSuccess ||
-      hipStreamSynchronize(stream) != hipSuccess)
+  if (ctx->host.to_host(dst, ld * elem, mc->staging, n * elem, m, stream, &status) != hipSuccess)
     return RNS8_BACKEND_FAILURE;
-  if (status != 0) return RNS8_RANGE_ERROR;
-  if (ctx->host.to_host(dst, ld * elem, mc->staging, n * elem, m, stream) != hipSuccess) return RNS8_BACKEND_FAILURE;
-  return RNS8_SUCCESS;
+  return status == 0 ? RNS8_SUCCESS : RNS8_RANGE_ERROR;
 }
 
 rns8_status export_device(rns8_context* ctx, const rns8_plan* plan, const rns8_matrix* C, void* d_dst, int64_t ld,
@@ -598,7 +598,9 @@ rns8_status oneshot_state(rns8_context* ctx, const rns8_gemm_desc& desc, Oneshot
 struct KeepOneshotOnSuccess {
   rns8_context* ctx;
   ~KeepOneshotOnSuccess() {
-    if (std::uncaught_exceptions() > 0) release_oneshot_cache(*ctx);
+    if (std::uncaught_exceptions() == 0) return;
+    (void)sync(ctx->stream);
+    release_oneshot_cache(*ctx);
   }
 };
 
@@ -649,9 +651,10 @@ rns8_status bounded_oneshot(rns8_context* ctx, const rns8_gemm_desc* desc, const
   if (st != RNS8_SUCCESS) return st;
   const KeepOneshotOnSuccess keep{ctx};
   OneshotState& s = *sp;
-  st = pack_native<T>(ctx, s.A, A, lda, 0, Source::Host, nullptr);
-  if (st == RNS8_SUCCESS) st = pack_native<T>(ctx, s.B, B, ldb, 0, Source::Host, nullptr);
-  if (st == RNS8_SUCCESS) st = gemm_rns(ctx, s.plan, s.A, s.B, s.C, s.ws, nullptr, true);
+  // uploads, packs and GEMM stay enqueued; the export waits for all of them
+  st = pack_native<T>(ctx, s.A, A, lda, 0, Source::HostQueued, nullptr);
+  if (st == RNS8_SUCCESS) st = pack_native<T>(ctx, s.B, B, ldb, 0, Source::HostQueued, nullptr);
+  if (st == RNS8_SUCCESS) st = gemm_rns(ctx, s.plan, s.A, s.B, s.C, s.ws, nullptr, false);
   if (st == RNS8_SUCCESS) {
     if (!valid_access(s.plan->desc.m, s.plan->desc.n, ldc)) st = RNS8_INVALID_ARGUMENT;
     else
@@ -660,6 +663,7 @@ rns8_status bounded_oneshot(rns8_context* ctx, const rns8_gemm_desc* desc, const
                                      is_signed ? RNS8_BOUNDED_I64 : RNS8_BOUNDED_U64, 1});
   }
   // a failed call, or one whose descriptor is not cacheable, keeps nothing
+  if (st != RNS8_SUCCESS) (void)sync(ctx->stream);
   if (st != RNS8_SUCCESS || !ctx->oneshot->reusable) release_oneshot_cache(*ctx);
   return st;
 }
@@ -674,10 +678,11 @@ rns8_status finite_oneshot(rns8_context* ctx, const rns8_gemm_desc* desc, rns8_s
   if (st != RNS8_SUCCESS) return st;
   const KeepOneshotOnSuccess keep{ctx};
   OneshotState& s = *sp;
-  st = pack_u8(ctx, s.A, modulus, A, lda, 0, Source::Host, nullptr);
-  if (st == RNS8_SUCCESS) st = pack_u8(ctx, s.B, modulus, B, ldb, 0, Source::Host, nullptr);
-  if (st == RNS8_SUCCESS) st = gemm_finite(ctx, s.plan, modulus, s.A, s.B, s.C, s.ws, nullptr, true);
+  st = pack_u8(ctx, s.A, modulus, A, lda, 0, Source::HostQueued, nullptr);
+  if (st == RNS8_SUCCESS) st = pack_u8(ctx, s.B, modulus, B, ldb, 0, Source::HostQueued, nullptr);
+  if (st == RNS8_SUCCESS) st = gemm_finite(ctx, s.plan, modulus, s.A, s.B, s.C, s.ws, nullptr, false);
   if (st == RNS8_SUCCESS) st = export_finite(ctx, s.plan, modulus, s.C, C, ldc, Source::Host, nullptr);
+  if (st != RNS8_SUCCESS) (void)sync(ctx->stream);
   if (st != RNS8_SUCCESS || !ctx->oneshot->reusable) release_oneshot_cache(*ctx);
   return st;
 }

@@ -137,7 +137,6 @@ struct rns8_matrix {
   std::size_t upload_bytes = 0;
   void* staging = nullptr;
   std::size_t staging_bytes = 0;
-  uint32_t* status = nullptr;
 };
 
 struct rns8_workspace {

@@ -78,7 +78,7 @@ HostStaging::~HostStaging() {
 hipError_t HostStaging::ensure() {
   for (int b = 0; b < 2; ++b) {
     if (!buf_[b]) {
-      const hipError_t e = hipHostMalloc(&buf_[b], kChunkBytes, hipHostMallocDefault);
+      const hipError_t e = hipHostMalloc(&buf_[b], kChunkBytes + kStatusBytes, hipHostMallocDefault);
       if (e != hipSuccess) {
         buf_[b] = nullptr;
         return e;
@@ -105,7 +105,8 @@ hipError_t HostStaging::to_device(void* dst, const void* src, std::size_t row_by
   char* const d = static_cast<char*>(dst);
   for (std::size_t i = 0; i < pieces.size(); ++i) {
     const Piece& p = pieces[i];
-    const int b = static_cast<int>(i & 1);
+    const int b = next_;
+    next_ ^= 1;
     // the DMA that last read this buffer must be finished before refilling it
     if ((e = hipEventSynchronize(done_[b])) != hipSuccess) return e;
     copy_piece(p, static_cast<char*>(buf_[b]), const_cast<char*>(static_cast<const char*>(src)), src_pitch, true);
@@ -119,18 +120,30 @@ hipError_t HostStaging::to_device(void* dst, const void* src, std::size_t row_by
 }
 
 hipError_t HostStaging::to_host(void* dst, std::size_t dst_pitch, const void* src, std::size_t row_bytes,
-                                int64_t rows, hipStream_t stream) {
+                                int64_t rows, hipStream_t stream, uint32_t* status) {
   if (rows <= 0 || row_bytes == 0) return hipSuccess;
   std::lock_guard<std::mutex> lock(mutex_);
   hipError_t e = ensure();
   if (e != hipSuccess) return e;
   const std::vector<Piece> pieces = plan_pieces(row_bytes, rows, kChunkBytes);
   const char* const s = static_cast<const char*>(src);
+  // The first transfers land in buffers that uploads may still read: those
+  // uploads are waited for (their events), whatever stream they run on.
+  for (int b = 0; b < 2; ++b)
+    if ((e = hipEventSynchronize(done_[b])) != hipSuccess) return e;
+  // The status word: behind the only piece, in the same transfer, or a
+  // transfer of its own in front of the first of several pieces.
+  const std::size_t total = row_bytes * static_cast<std::size_t>(rows);
+  const std::size_t with_status = status && pieces.size() == 1 ? sizeof(*status) : 0;
+  char* const status_at = static_cast<char*>(buf_[0]) + (with_status ? total : kChunkBytes);
+  if (status && !with_status &&
+      (e = hipMemcpyAsync(status_at, s + total, sizeof(*status), hipMemcpyDeviceToHost, stream)) != hipSuccess)
+    return e;
   auto issue = [&](std::size_t i) -> hipError_t {
     const Piece& p = pieces[i];
     const int b = static_cast<int>(i & 1);
     const std::size_t off = static_cast<std::size_t>(p.row0) * row_bytes + p.col0;
-    hipError_t err = hipMemcpyAsync(buf_[b], s + off, static_cast<std::size_t>(p.nrows) * p.bytes,
+    hipError_t err = hipMemcpyAsync(buf_[b], s + off, static_cast<std::size_t>(p.nrows) * p.bytes + with_status,
                                     hipMemcpyDeviceToHost, stream);
     if (err == hipSuccess) err = hipEventRecord(done_[b], stream);
     return err;
@@ -142,6 +155,10 @@ hipError_t HostStaging::to_host(void* dst, std::size_t dst_pitch, const void* sr
     if (i + 1 < pieces.size() && (e = issue(i + 1)) != hipSuccess) return e;
     const int b = static_cast<int>(i & 1);
     if ((e = hipEventSynchronize(done_[b])) != hipSuccess) return e;
+    if (status && i == 0) {
+      std::memcpy(status, status_at, sizeof(*status));
+      if (*status != 0) return hipStreamSynchronize(stream);
+    }
     copy_piece(pieces[i], static_cast<char*>(buf_[b]), static_cast<char*>(dst), dst_pitch, false);
   }
   return hipSuccess;

@@ -31,15 +31,20 @@ class HostStaging {
                        hipStream_t stream);
 
   // dst (host) row r at dst + r * dst_pitch receives row r of the packed
-  // device matrix src. Returns when dst holds the data.
+  // device matrix src. Returns when dst holds the data. With `status`, the
+  // word behind the matrix (src + rows * row_bytes) is read first and, unless
+  // it is zero, dst stays untouched. It travels with the matrix where both fit
+  // one buffer.
   hipError_t to_host(void* dst, std::size_t dst_pitch, const void* src, std::size_t row_bytes, int64_t rows,
-                     hipStream_t stream);
+                     hipStream_t stream, uint32_t* status = nullptr);
 
  private:
+  static constexpr std::size_t kStatusBytes = 64;  // room for a status word behind a full chunk
   hipError_t ensure();
 
   std::mutex mutex_;
   void* buf_[2] = {nullptr, nullptr};
+  int next_ = 0;  // buffer the next upload starts with, so that back-to-back uploads overlap too
   hipEvent_t done_[2] = {nullptr, nullptr};
 };
 
