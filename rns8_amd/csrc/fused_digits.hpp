@@ -39,6 +39,9 @@
 // centered residues [slice][row][16 columns x groups] in the workspace; a
 // finalize adds the slices and writes C's planes. Weights and residues take at
 // most kMaxPart bytes each: larger K or m run in parts.
+// (Compiled as part of fused_skinny.hip.)
+#pragma once
+
 #include <algorithm>
 #include <type_traits>
 
@@ -48,6 +51,7 @@
 #include "plane_consts.hpp"
 
 namespace rns8x {
+namespace digits {
 namespace {
 
 constexpr int kWaves = 4;
@@ -425,4 +429,5 @@ hipError_t launch_fused_digits(const FusedArgs& f, hipStream_t stream) {
   return hipSuccess;
 }
 
+}  // namespace digits
 }  // namespace rns8x

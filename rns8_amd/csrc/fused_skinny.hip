@@ -6,7 +6,7 @@
 // hip_direct_gemm_tiled_kernels.cuh:298-432).
 //
 // Products whose planes x columns fill few 16-column groups run in
-// fused_digits.hip instead (fused_digits_shape says which).
+// fused_digits.hpp instead (fused_digits_shape says which).
 //
 // The packed route writes every residue plane of A to HBM and reads it back:
 // at 8192 x 1 x 8192 with 9 planes that is 537 MB read, 604 MB written and
@@ -55,6 +55,7 @@
 #include <type_traits>
 
 #include "dma.hpp"
+#include "fused_digits.hpp"
 #include "int_ops.hpp"
 #include "kernels.hpp"
 #include "plane_consts.hpp"
@@ -383,8 +384,8 @@ bool fused_skinny_shape(int64_t m, int64_t n, int64_t k, uint32_t nplanes, Fused
   out.skinny = 1;
   out.bt_bytes = bt;
   // (which products are accepted stays this form's rule)
-  FusedShape digits;
-  if (fused_digits_shape(m, n, k, nplanes, digits)) out = digits;
+  FusedShape form;
+  if (digits::fused_digits_shape(m, n, k, nplanes, form)) out = form;
   return true;
 }
 
