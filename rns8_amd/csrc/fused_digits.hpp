@@ -21,7 +21,10 @@
 // 97 us for 537 MB (5.5 TB/s; a plain read of as much reaches 5.6-5.7), 8 us
 // more with the weights and the finalize; reducing every element to every
 // plane's residue in registers (fused_skinny.hip) took 147 us in all, and more
-// with every plane. Non-temporal loads of A: 114 against 123 us; 1024 instead
+// with every plane. Non-temporal loads of A: 114 against 123 us,
+// but only where rows start on cache lines: a line that two steps share was
+// then fetched twice (4498 x 4 x 1043 at 9 planes 26.7 us, ordinary loads 22.2;
+// 989 x 10 x 6774 55.5 and 48.1); 1024 instead
 // of 512 workgroups: 106 against 114; two or four lines of a row per step: 111
 // and 118 (more bytes per row in flight, fewer rows).
 //
@@ -77,6 +80,7 @@ struct DigitsArgs {
   uint32_t slot_row;
   uint32_t columns, n;  // column q is column q % n of plane q / n
   uint32_t slice0, k_slice, row_groups;
+  uint32_t whole_lines;  // every row starts on a 128-byte line: a step reads whole lines once
 };
 
 // Centered residue of the 64-bit value (hi:lo) mod mc.m (pack.hip's wide
@@ -178,7 +182,10 @@ __global__ __launch_bounds__(kThreads, 2) void fused_digits_kernel(DigitsArgs a)
     const v4i ra = buffer_rsrc(a_at, live ? a_left : 0);
     const v4i rw = buffer_rsrc(w_at, live ? (G - 1) * static_cast<int64_t>(a.w_stride) + kStepBytes : 0);
 #pragma unroll
-    for (int i = 0; i < kABlocks; ++i) dma16_stream(lds_a + stage * kStageA + 1024u * i, a_voff[i], ra);
+    for (int i = 0; i < kABlocks; ++i) {
+      if (a.whole_lines) dma16_stream(lds_a + stage * kStageA + 1024u * i, a_voff[i], ra);
+      else dma16(lds_a + stage * kStageA + 1024u * i, a_voff[i], ra);
+    }
 #pragma unroll
     for (int i = 0; i < kWBlocks; ++i) dma16(lds_w + stage * kStageW + 1024u * i, w_voff[i], rw);
     a_at += 8 * kStepK;
@@ -399,6 +406,7 @@ hipError_t launch_fused_digits(const FusedArgs& f, hipStream_t stream) {
       a.k_slice = static_cast<uint32_t>(p.k_slice);
       a.row_groups = (rows + kGroupRows - 1) / kGroupRows;
       a.w = f.ws;
+      a.whole_lines = (reinterpret_cast<uintptr_t>(f.a) % 128u == 0 && f.lda % kStepK == 0) ? 1u : 0u;
       a.slots = slots;
       auto run = [&](auto sg, auto g) {
         hipLaunchKernelGGL((fused_digits_kernel<decltype(sg)::value, decltype(g)::value>),
