@@ -342,6 +342,8 @@ bool fused_digits_shape(int64_t m, int64_t n, int64_t k, uint32_t nplanes, Fused
   //     three launches cost more than they save (8000 x 5 x 300, 3 planes 12.8
   //     / 15.3); at 5 and 6 only below 2^18 elements of A (128 x 5 x 256,
   //     6 planes 13.9 / 14.3; 512 x 3 x 512, 5 planes 19.1 / 13.3).
+  //     Above 2^23 elements five planes' arithmetic hides behind the residue
+  //     form's loads (5748 x 5 x 6620, 5 planes 79 / 89).
   //   3 groups <= 2 planes: while A is small enough to leave the residue form
   //     idle CUs and long enough to amortize the launches (2000 x 9 x 1000, 9
   //     planes 50 / 29; 2000 x 8 x 1000, 5 planes 33 / 21; but 8000 x 8 x 300,
@@ -352,7 +354,8 @@ bool fused_digits_shape(int64_t m, int64_t n, int64_t k, uint32_t nplanes, Fused
   // 16 x 4 x 100000 60 / 98; 64 x 2 x 8000 53 / 17, 16 x 1 x 100000 60 / 43).
   const int64_t groups = groups_of(nplanes, n), work = m * k;
   if (m < 16 * (2 * groups - 1) || groups > kMaxGroups || nplanes < 5) return false;
-  const bool few = nplanes >= 2 * groups + 1 && (nplanes >= 7 || work >= (int64_t{1} << 18));
+  const bool few = nplanes >= 2 * groups + 1 &&
+                   (nplanes >= 7 || (work >= (int64_t{1} << 18) && work <= (int64_t{1} << 23)));
   const bool mid = 3 * groups <= 2 * nplanes && k >= 512 && k <= 8192 && work >= (int64_t{1} << 18) &&
                    work <= (int64_t{1} << 23);
   if (!few && !mid) return false;
