@@ -197,14 +197,15 @@ __global__ __launch_bounds__(kThreads, 4) void native_axes_kernel(const uint64_t
     if (threadIdx.x == 0) {
       for (int w = 1; w < kWaves; ++w) best = wave_best[w] > best ? wave_best[w] : best;
       // The block's maximum is in before its ticket is drawn (the wait), so
-      // the block that draws the last one reads everybody's. It leaves the
-      // ticket as it found it.
+      // the block that draws the last one reads everybody's. The count wraps
+      // to zero by itself: packs of one matrix that overlap (a caller's
+      // error, and their maxima may mix) still draw whole multiples of
+      // row_blocks, so the next pack starts from a clean ticket.
       const u64 before = __hip_atomic_fetch_max(&ticket->best, best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       asm volatile("s_waitcnt vmcnt(0)" ::"v"(before) : "memory");
-      if (__hip_atomic_fetch_add(&ticket->drawn, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == row_blocks - 1) {
+      if (atomicInc(&ticket->drawn, row_blocks - 1) == row_blocks - 1) {
         words[0] = __hip_atomic_exchange(&ticket->best, u64{0}, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         for (int i = 1; i < 8; ++i) words[i] = 0;
-        __hip_atomic_store(&ticket->drawn, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     }
     return;

@@ -35,7 +35,8 @@ hipError_t launch_pack_native(const PackArgs& args, hipStream_t stream);
 // Per-row and per-column summaries of a rows x cols native operand (row
 // stride ld elements) into out_rows / out_cols, and its max |x| into
 // words[0] (words[1..7] zero). ticket: zero before the matrix's first launch;
-// every launch leaves it zero. Launches on one ticket are ordered.
+// every launch leaves it zero, overlapping ones (of one row count) once all of
+// them are done. Launches on one ticket are to be ordered.
 struct ProofTicket {
   unsigned long long best;
   uint32_t drawn, unused;

@@ -56,3 +56,39 @@ def test_axes_edges(gpu_ctx, signed, rows, cols, ld):
             assert len(got) == len(axes)
             for i, (g, w) in enumerate(zip(got, axes)):
                 assert all(g[f] == getattr(w, f) for f in FIELDS), (turn, i, g)
+
+
+def test_pack_after_overlapping_packs(gpu_ctx):
+    """Packs of one matrix on two streams at once are a caller's error and may
+    spoil their own proofs, but not the next pack's: with an ordered pack
+    behind them, of smaller values, the matrix's maximum and summaries are that
+    pack's."""
+    ctx = gpu_ctx
+    rows, cols = 6000, 40
+    pack = r.lib().rns8_mi355x_pack_i64_device
+    M = r.Matrix(ctx, r.matrix_desc(rows, cols, r.EXACT_WIDE_SIGNED, r.BOUND_NONE, 20))
+    big = inputs.splitmix64(91, rows * cols).reshape(rows, cols).view(np.int64)
+    small = big >> np.int64(40)
+    d_big, d_small = hip.malloc(big.nbytes), hip.malloc(small.nbytes)
+    streams = [hip.stream_create(), hip.stream_create()]
+    try:
+        hip.to_device(d_big, big)
+        hip.to_device(d_small, small)
+        for turn in range(4):
+            for _ in range(20):
+                for s in streams:
+                    r.check(pack(ctx.ptr, M.ptr, ctypes.c_void_p(d_big), cols, 0, ctypes.c_void_p(s)), "pack")
+            hip.synchronize()
+            r.check(pack(ctx.ptr, M.ptr, ctypes.c_void_p(d_small), cols, 0, None), "pack")
+            hip.synchronize()
+            bound, kind, got_rows, got_cols = M.exact_proof(ctx)
+            assert kind == r.EXACT_AXES_NATIVE and bound == int(np.abs(small).max()), turn
+            for axis, got in ((1, got_rows), (0, got_cols)):
+                want = small.sum(axis=axis)
+                assert [g["sum"] for g in got] == [int(v) for v in want], turn
+    finally:
+        hip.synchronize()
+        for s in streams:
+            hip.stream_destroy(s)
+        hip.free(d_big)
+        hip.free(d_small)
