@@ -1084,7 +1084,8 @@ rns8_status rns8_create_matrix(rns8_context* ctx, const rns8_matrix_desc* desc, 
       return RNS8_BACKEND_FAILURE;
     }
     // exact-wide matrices: the device proof (two sets of axis records and the
-    // pack proof's ticket, zeroed below with the planes) and its event
+    // pack proof's ticket, zeroed below with the planes, and its partials) and
+    // its event
     const uint64_t proof_bytes = rns8_matrix::proof_bytes(m->desc.rows, m->desc.cols);
     if (exact_wide(desc->semantics) &&
         (hipMalloc(reinterpret_cast<void**>(&m->proof_device), proof_bytes) != hipSuccess ||

@@ -7,7 +7,8 @@
 //   where its values were read: the values stay in registers (up to 2048 of a
 //   row, 1024 of a column; longer axes read them again) for the deviation sums
 //   around that centre, and nothing goes through partial summaries. The last
-//   row block to finish writes the operand's max |x|.
+//   row block to finish writes the operand's max |x|. Few long axes, and large
+//   operands, run in the tile form instead (native_axes_tiled).
 // * product_axes: the cell bounds of C = A x B from A's row records and B's
 //   column records, reduced per row (one wave per row) and per column (one
 //   wave per column), and C's bound min(k maxA maxB, max cell).
@@ -119,8 +120,7 @@ __device__ __forceinline__ v2u64 load_pair(const uint64_t* base, Off off, int64_
 // its loads and reductions. At 2048 x 2048 it takes 24 us, at 500 x 701 10 us;
 // the four launches it replaces (two passes over 64 x 64 LDS tiles, each
 // followed by a merge of the tiles' partials) took 14 + 6 + 11 + 5 and 20 us.
-// Only operands of few columns and more rows than a column block holds read
-// worse (5000 x 300: 34 against 29 us).
+// Where that is not so, the tile form below runs (native_axes_tiled).
 // kVec: 16-byte loads; kFar: 64-bit lane offsets (row strides from 2^21 on).
 template <bool Signed, bool kVec, bool kFar>
 __global__ __launch_bounds__(kThreads, 4) void native_axes_kernel(const uint64_t* __restrict__ src, int64_t rows,
@@ -316,6 +316,183 @@ __global__ __launch_bounds__(kThreads, 4) void native_axes_kernel(const uint64_t
   }
 }
 
+// ---- the tile form: operands with few long axes, and large ones -------------
+// (native_axes_tiled says which, with both forms' times). Two passes over 64 x
+// 64 tiles staged in LDS, each followed by a merge of the tiles' partials: four
+// launches, but a long axis is spread over the chip, and each pass reads the
+// operand once for both directions.
+
+constexpr int kTile = 64;
+constexpr int64_t kMaxGridY = 65535;
+// Elements of a half-tile run read per batch: the batch's LDS reads issue
+// together and one wait covers them (a rolled loop waits on every read).
+constexpr int kWalkBatch = 8;
+
+// f(elem(j)) for j in [j0, j1): whole 32-element runs (every run of a full
+// tile) in batches of kWalkBatch reads, ragged ones one element at a time.
+template <typename E, typename F>
+__device__ __forceinline__ void walk_run(int j0, int j1, E elem, F f) {
+  if (j1 - j0 == kTile / 2) {
+#pragma unroll 1
+    for (int b = 0; b < kTile / 2; b += kWalkBatch) {
+      u64 v[kWalkBatch];
+#pragma unroll
+      for (int e = 0; e < kWalkBatch; ++e) v[e] = elem(j0 + b + e);
+#pragma unroll
+      for (int e = 0; e < kWalkBatch; ++e) f(v[e]);
+    }
+  } else {
+    for (int j = j0; j < j1; ++j) f(elem(j));
+  }
+}
+
+// One pass over the 64 x 64 tiles of a rows x cols operand (row stride ld).
+// Block (x, y) takes tile column x and tile rows y, y + gridDim.y, ...; each
+// lane holds its 16 elements of the next tile in registers, loaded while the
+// current tile is summarized. Partials: row r of tile column x at
+// row_part[x * rows + r], column c of tile row y at col_part[y * cols + c].
+// Pass 1 (Dev = false) also clears the result's 8 proof words (block (0,
+// 0)), which the finishing launch fills; pass 2 reads the axis centres from
+// the records pass 1 finished.
+template <bool Signed, bool Dev>
+__global__ __launch_bounds__(256) void tiled_axes_pass(const uint64_t* __restrict__ src, int64_t rows, int64_t cols,
+                                                       int64_t ld, AxisPartial* __restrict__ row_part,
+                                                       AxisPartial* __restrict__ col_part,
+                                                       const AxisRecord* __restrict__ row_rec,
+                                                       const AxisRecord* __restrict__ col_rec, u64* __restrict__ words) {
+  // the tile as 32-bit halves at a row stride of 65 words: row and column
+  // reads are both free of bank conflicts
+  __shared__ uint32_t tile_lo[kTile][kTile + 1], tile_hi[kTile][kTile + 1];
+  __shared__ AxisPartial second[2][kTile];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t c0 = static_cast<int64_t>(blockIdx.x) * kTile;
+  const int nc = static_cast<int>(cols - c0 < kTile ? cols - c0 : kTile);
+  if (!Dev && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 8) words[threadIdx.x] = 0;
+  // waves 0, 1: rows (lane = row) over column halves; waves 2, 3: columns
+  // (lane = column) over row halves
+  const bool by_row = wave < 2;
+  const int half = wave & 1;
+  i128 col_centre = 0;
+  if (Dev && !by_row && lane < nc) col_centre = record_centre(col_rec[c0 + lane]);
+  const int64_t tiles_y = (rows + kTile - 1) / kTile;
+  // rows wave, wave + 4, ..., wave + 60 of a tile, column c0 + lane
+  u64 next[kTile / 4];
+  auto fetch = [&](int64_t ty) {
+    const int64_t r0 = ty * kTile;
+    const int nr = static_cast<int>(rows - r0 < kTile ? rows - r0 : kTile);
+#pragma unroll
+    for (int q = 0; q < kTile / 4; ++q) {
+      const int i = wave + 4 * q;
+      next[q] = lane < nc && i < nr ? src[(r0 + i) * ld + c0 + lane] : 0;
+    }
+  };
+  if (static_cast<int64_t>(blockIdx.y) < tiles_y) fetch(blockIdx.y);
+  for (int64_t ty = blockIdx.y; ty < tiles_y; ty += gridDim.y) {
+    const int64_t r0 = ty * kTile;
+    const int nr = static_cast<int>(rows - r0 < kTile ? rows - r0 : kTile);
+    __syncthreads();  // the previous tile's readers are done
+#pragma unroll
+    for (int q = 0; q < kTile / 4; ++q) {
+      tile_lo[wave + 4 * q][lane] = static_cast<uint32_t>(next[q]);
+      tile_hi[wave + 4 * q][lane] = static_cast<uint32_t>(next[q] >> 32);
+    }
+    __syncthreads();
+    if (ty + gridDim.y < tiles_y) fetch(ty + gridDim.y);
+    const int axes = by_row ? nr : nc, len = by_row ? nc : nr;
+    const int j0 = half * 32, j1 = j0 + 32 < len ? j0 + 32 : len;
+    AxisPartial p = empty_partial();
+    auto row_elem = [&](int j) { return (static_cast<u64>(tile_hi[lane][j]) << 32) | tile_lo[lane][j]; };
+    auto col_elem = [&](int j) { return (static_cast<u64>(tile_hi[j][lane]) << 32) | tile_lo[j][lane]; };
+    if (lane < axes) {
+      if (!Dev) {
+        PartialAcc acc;
+        if (by_row)
+          walk_run(j0, j1, row_elem, [&](u64 x) { acc.add(x, Signed); });
+        else
+          walk_run(j0, j1, col_elem, [&](u64 x) { acc.add(x, Signed); });
+        p = acc.partial();
+      } else {
+        const i128 centre = by_row ? record_centre(row_rec[r0 + lane]) : col_centre;
+        DeviationAcc acc;
+        if (by_row)
+          walk_run(j0, j1, row_elem, [&](u64 x) { acc.add(deviation(x, centre, Signed)); });
+        else
+          walk_run(j0, j1, col_elem, [&](u64 x) { acc.add(deviation(x, centre, Signed)); });
+        p.sum = acc.value();
+      }
+    }
+    if (half == 1) second[by_row ? 0 : 1][lane] = p;
+    __syncthreads();
+    if (half == 0 && lane < axes) {
+      partial_merge(p, second[by_row ? 0 : 1][lane]);
+      if (by_row)
+        row_part[static_cast<int64_t>(blockIdx.x) * rows + r0 + lane] = p;
+      else
+        col_part[ty * cols + c0 + lane] = p;
+    }
+  }
+}
+
+// Merges each axis's partials (rows first, then columns): pass 1 writes the
+// records and the operand's max |x| (words[0], an atomic max per block);
+// pass 2 adds the deviation sums. A block takes 32 axes; its 8 thread groups
+// each merge every 8th partial of them, and group 0 merges the 8 results.
+template <bool Signed, bool Dev>
+__global__ __launch_bounds__(256) void tiled_axes_finish(const AxisPartial* __restrict__ row_part,
+                                                          const AxisPartial* __restrict__ col_part, int64_t rows,
+                                                          int64_t cols, AxisRecord* __restrict__ out_rows,
+                                                          AxisRecord* __restrict__ out_cols, u64* __restrict__ words) {
+  constexpr int kAxes = 32, kGroups = 8;
+  __shared__ AxisPartial part_of[kGroups][kAxes];
+  __shared__ u64 block_max;
+  const int64_t tiles_x = (cols + kTile - 1) / kTile, tiles_y = (rows + kTile - 1) / kTile;
+  const int a = threadIdx.x % kAxes, g = threadIdx.x / kAxes;
+  if (threadIdx.x == 0) block_max = 0;
+  u64 best = 0;
+  for (int64_t base = static_cast<int64_t>(blockIdx.x) * kAxes; base < rows + cols;
+       base += static_cast<int64_t>(gridDim.x) * kAxes) {
+    const int64_t i = base + a;
+    const bool valid = i < rows + cols, is_row = i < rows;
+    const int64_t axis = is_row ? i : i - rows, stride = is_row ? rows : cols, parts = is_row ? tiles_x : tiles_y;
+    AxisPartial p = empty_partial();
+    if (valid) {
+      const AxisPartial* const part = (is_row ? row_part : col_part) + axis;
+      for (int64_t t = g; t < parts; t += kGroups) {
+        if (!Dev)
+          partial_merge(p, part[t * stride]);
+        else
+          p.sum += part[t * stride].sum;
+      }
+    }
+    __syncthreads();  // the previous round's readers are done
+    part_of[g][a] = p;
+    __syncthreads();
+    if (g == 0 && valid) {
+      for (int h = 1; h < kGroups; ++h) {
+        if (!Dev)
+          partial_merge(p, part_of[h][a]);
+        else
+          p.sum += part_of[h][a].sum;
+      }
+      AxisRecord* const rec = (is_row ? out_rows : out_cols) + axis;
+      if (!Dev) {
+        // the groups' partials start empty (hi = not_lo = 0 are neutral)
+        const AxisRecord r = native_record(p, static_cast<u64>(is_row ? cols : rows), Signed);
+        *rec = r;
+        if (is_row) best = r.max_magnitude[0] > best ? r.max_magnitude[0] : best;
+      } else {
+        put_u128(rec->deviation_sum, p.sum);
+      }
+    }
+  }
+  if (!Dev) {
+    if (best) atomicMax(reinterpret_cast<unsigned long long*>(&block_max), static_cast<unsigned long long>(best));
+    __syncthreads();
+    if (threadIdx.x == 0 && block_max)
+      atomicMax(reinterpret_cast<unsigned long long*>(words), static_cast<unsigned long long>(block_max));
+  }
+}
+
 struct ProductArgs {
   const AxisRecord* arows;  // m records (unused for a uniform A)
   const AxisRecord* bcols;  // n records (unused for a uniform B)
@@ -423,12 +600,49 @@ unsigned blocks_for(int64_t items, int64_t per_block, int64_t cap) {
 
 }  // namespace
 
+namespace {
+
+hipError_t launch_tiled_axes(const uint64_t* src, int64_t rows, int64_t cols, int64_t ld, bool is_signed,
+                             AxisRecord* out_rows, AxisRecord* out_cols, uint64_t* words, AxisPartial* partials,
+                             hipStream_t stream) {
+  const int64_t tiles_x = (cols + kTile - 1) / kTile, tiles_y = (rows + kTile - 1) / kTile;
+  if (tiles_x > 0x7FFFFFFFll) return hipErrorInvalidValue;
+  AxisPartial* const row_part = partials;
+  AxisPartial* const col_part = partials + rows * tiles_x;
+  // two tiles per block where there are enough: one loads while the other is summarized
+  const int64_t gy = tiles_x * tiles_y >= 2048 ? (tiles_y + 1) / 2 : tiles_y;
+  const dim3 grid(static_cast<unsigned>(tiles_x), static_cast<unsigned>(gy < kMaxGridY ? gy : kMaxGridY));
+  const unsigned fin = blocks_for(rows + cols, 32, 4096);
+  auto run = [&](auto sgn) {
+    constexpr bool S = decltype(sgn)::value;
+    hipLaunchKernelGGL((tiled_axes_pass<S, false>), grid, dim3(256), 0, stream, src, rows, cols, ld, row_part,
+                       col_part, out_rows, out_cols, words);
+    hipLaunchKernelGGL((tiled_axes_finish<S, false>), dim3(fin), dim3(256), 0, stream, row_part, col_part, rows,
+                       cols, out_rows, out_cols, words);
+    hipLaunchKernelGGL((tiled_axes_pass<S, true>), grid, dim3(256), 0, stream, src, rows, cols, ld, row_part,
+                       col_part, out_rows, out_cols, words);
+    hipLaunchKernelGGL((tiled_axes_finish<S, true>), dim3(fin), dim3(256), 0, stream, row_part, col_part, rows,
+                       cols, out_rows, out_cols, words);
+  };
+  if (is_signed)
+    run(std::true_type{});
+  else
+    run(std::false_type{});
+  return hipGetLastError();
+}
+
+}  // namespace
+
 hipError_t launch_native_axes(const void* src, int64_t rows, int64_t cols, int64_t ld, bool is_signed,
                               xa::AxisRecord* out_rows, xa::AxisRecord* out_cols, uint64_t* words,
-                              ProofTicket* ticket, hipStream_t stream) {
+                              ProofTicket* ticket, xa::AxisPartial* partials, hipStream_t stream) {
   if (!src || !out_rows || !out_cols || !words || !ticket || rows <= 0 || cols <= 0 || ld < cols)
     return hipErrorInvalidValue;
   const uint64_t* s = static_cast<const uint64_t*>(src);
+  if (native_axes_tiled(rows, cols)) {
+    if (!partials) return hipErrorInvalidValue;
+    return launch_tiled_axes(s, rows, cols, ld, is_signed, out_rows, out_cols, words, partials, stream);
+  }
   const unsigned rb = blocks_for(rows, kWaves, kMaxBlocks);
   // whole groups of 16 column blocks (see the kernel's numbering)
   const unsigned cb = blocks_for((cols + kColsPerBlock - 1) / kColsPerBlock, 16, kMaxBlocks / 16) * 16;

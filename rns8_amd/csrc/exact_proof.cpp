@@ -35,7 +35,7 @@ rns8_status read_words(const uint64_t* src, hipStream_t stream, uint64_t (&w)[4]
 rns8_status prove_native(const rns8_matrix& m, const void* src, int64_t ld, bool is_signed, hipStream_t stream) {
   const uint32_t t = m.proof_set ^ 1u;
   return launch_native_axes(src, m.desc.rows, m.desc.cols, ld, is_signed, m.proof_rows(t), m.proof_cols(t),
-                            m.proof_words(t), m.proof_ticket(), stream) == hipSuccess
+                            m.proof_words(t), m.proof_ticket(), m.proof_partials(), stream) == hipSuccess
              ? RNS8_SUCCESS
              : RNS8_BACKEND_FAILURE;
 }

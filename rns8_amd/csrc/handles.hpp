@@ -119,11 +119,12 @@ struct rns8_matrix {
   uint32_t lazy_rows = 0, lazy_cols = 0;  // rns8x::xa::AxisKind of a lazy proof's snapshot
   uint64_t lazy_k = 0;
   // [words set 0 (8)] [words set 1 (8)] [set 0 rows] [set 0 cols] [set 1
-  // rows] [set 1 cols] [the pack proof's ticket]
+  // rows] [set 1 cols] [the pack proof's ticket] [its tile form's partials]
   uint8_t* proof_device = nullptr;
   hipEvent_t proof_event = nullptr;
   static uint64_t proof_bytes(int64_t rows, int64_t cols) {
-    return 128u + 2u * static_cast<uint64_t>(rows + cols) * sizeof(rns8x::xa::AxisRecord) + sizeof(rns8x::ProofTicket);
+    return 128u + 2u * static_cast<uint64_t>(rows + cols) * sizeof(rns8x::xa::AxisRecord) + sizeof(rns8x::ProofTicket) +
+           static_cast<uint64_t>(rns8x::native_axes_partials(rows, cols)) * sizeof(rns8x::xa::AxisPartial);
   }
   uint64_t* proof_words(uint32_t set) const { return reinterpret_cast<uint64_t*>(proof_device) + 8u * set; }
   rns8x::xa::AxisRecord* proof_rows(uint32_t set) const {
@@ -131,6 +132,9 @@ struct rns8_matrix {
   }
   rns8x::xa::AxisRecord* proof_cols(uint32_t set) const { return proof_rows(set) + desc.rows; }
   rns8x::ProofTicket* proof_ticket() const { return reinterpret_cast<rns8x::ProofTicket*>(proof_rows(2)); }
+  rns8x::xa::AxisPartial* proof_partials() const {
+    return reinterpret_cast<rns8x::xa::AxisPartial*>(proof_ticket() + 1);
+  }
   // cached staging buffers (export is logically const, reference
   // api_export.cpp:276-287 keeps the same kind of cache on the matrix)
   void* upload = nullptr;

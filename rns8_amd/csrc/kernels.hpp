@@ -41,9 +41,34 @@ struct ProofTicket {
   unsigned long long best;
   uint32_t drawn, unused;
 };
+// partials: scratch for native_axes_partials(rows, cols) partials.
 hipError_t launch_native_axes(const void* src, int64_t rows, int64_t cols, int64_t ld, bool is_signed,
                               xa::AxisRecord* out_rows, xa::AxisRecord* out_cols, uint64_t* words,
-                              ProofTicket* ticket, hipStream_t stream);
+                              ProofTicket* ticket, xa::AxisPartial* partials, hipStream_t stream);
+// Whether an operand's summaries run in the tile form (four launches over 64 x
+// 64 tiles) instead of one launch that takes each axis whole. Times of the
+// proof's kernels, one launch / tile form in us:
+//   * few long axes: one block walks a long axis, about 4.3 us per 1024 values
+//     (16384 x 8: 70 / 37, 8 x 65536: 270 / 94, 1048576 x 8: 3530 / 1390, 8192
+//     x 384: 43.5 / 37, 640 x 16384: 78.6 / 78.4; but 8192 x 768: 47 / 50, 768
+//     x 16384: 81 / 86, and 6144 x 64: 32 / 24 and three more launches);
+//   * operands past the caches whose rows (above 2048 values) and columns (above
+//     1024) do not stay in registers: four reads against two (8192^2: 384 / 312,
+//     12288^2: 948 / 695, 4096 x 6144: 142 / 120, 1536 x 16384: 147 / 133; but
+//     4096^2: 84 / 85, 1536 x 8192: 66 / 76, 16384 x 2048: 130 / 171, 1024 x
+//     65536: 393 / 463);
+//   * very long columns: 65536 x 1024: 477 / 421, 65536 x 1280: 601 / 508.
+inline bool native_axes_tiled(int64_t rows, int64_t cols) {
+  const int64_t longer = rows > cols ? rows : cols, shorter = rows > cols ? cols : rows;
+  if (longer >= 8192 && shorter <= (longer >= 32768 ? 768 : 640)) return true;
+  if (rows >= 65536) return true;
+  return rows > 1024 && cols > 2048 && rows > (int64_t{20} << 20) / cols;
+}
+// The tile form's scratch: a partial per row and tile column, then one per
+// column and tile row.
+inline int64_t native_axes_partials(int64_t rows, int64_t cols) {
+  return native_axes_tiled(rows, cols) ? rows * ((cols + 63) / 64) + cols * ((rows + 63) / 64) : 0;
+}
 // The carried summaries of C = A x B (m x n, inner k): per-row and
 // per-column maxima and sums of the cell bounds from A's m row records and
 // B's n column records (kinds: xa::AxisKind; a uniform side reads no

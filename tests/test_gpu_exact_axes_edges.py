@@ -1,7 +1,9 @@
 """The pack-time summaries of exact-wide operands at the edges of the summary
 kernel's split: rows of one wave and of eight, column groups of eight,
 register chunks of 512 rows and 2048 columns held and re-read, odd row
-strides, and two packs into one matrix in a row (the second one's maximum must
+strides, row strides that need 64-bit lane offsets (2^21), long axes of either
+direction that run in the tile form (ragged tiles, one and several tile
+columns), and two packs into one matrix in a row (the second one's maximum must
 not see the first one's). Every field against oracle/exact_range.py."""
 from __future__ import annotations
 
@@ -23,7 +25,10 @@ FIELDS = ("max_magnitude", "absolute_sum", "sum", "minimum", "maximum", "deviati
 @pytest.mark.parametrize(
     "rows,cols,ld",
     [(1, 1, 1), (9, 8, 8), (8, 9, 11), (513, 17, 18), (1025, 7, 7), (511, 16, 16), (2050, 3, 4), (1024, 130, 130),
-     (3, 2047, 2048), (2, 2049, 2049), (17, 4100, 4100)],
+     (3, 2047, 2048), (2, 2049, 2049), (17, 4100, 4100),
+     (3, 70, 1 << 21), (3, 5000, 1 << 21), (8191, 3, 3), (5, 8191, 8191),
+     # few axes of 8192 values and more: the tile form
+     (1, 8192, 8192), (8192, 1, 1), (70, 8200, 8203), (8257, 65, 66), (2, 65700, 65700)],
 )
 def test_axes_edges(gpu_ctx, signed, rows, cols, ld):
     ctx = gpu_ctx
@@ -39,9 +44,8 @@ def test_axes_edges(gpu_ctx, signed, rows, cols, ld):
             x[-1, -1] = np.uint64((1 << 63) - 1)
         if signed:
             x = x.view(np.int64)
-        staged = np.zeros((rows, ld), dtype=x.dtype)
-        staged[:, :cols] = x
-        staged[:, cols:] = -1 if signed else 0xFFFFFFFFFFFFFFFF  # padding is not part of the operand
+        staged = np.full((rows, ld), -1 if signed else 0xFFFFFFFFFFFFFFFF, dtype=x.dtype)
+        staged[:, :cols] = x  # padding is not part of the operand
         d = hip.malloc(staged.nbytes)
         try:
             hip.to_device(d, staged)

@@ -11,10 +11,11 @@ the library takes with them against the same oracle:
 * native summaries of device-pointer and host-array packs, int64 and uint64
   over the full ranges with the extremes placed, strided sources, shapes of
   one to several 64 x 64 tiles with ragged edges, and prefixes above and
-  below 9 (where the pack reads max |x| back before writing); and 4100 x
-  2050 and 140000 x 8 operands, whose tiles run two tile rows per block and
-  whose finishing launch strides over its axes (checked against numpy, in a
-  range where int64 is exact);
+  below 9 (where the pack reads max |x| back before writing); and, checked
+  against numpy in a range where int64 is exact, operands of 4100 x 2050 (one
+  launch, axes longer than the registers hold), 5130 x 4110 and 140000 x 8 (the
+  tile form: two tile rows per block, a finishing launch that strides over its
+  axes) and 770 x 65560 (one launch whose column blocks stride);
 * the carried summaries of a product, computed lazily from the snapshot of
   its operands' summaries, also over 33000 rows (more rows than waves);
 * decisions at the range threshold that the worst case k * maxA * maxB
@@ -124,19 +125,21 @@ def test_native_summaries(gpu_ctx, signed, device, shape, ld_pad):
 
 
 @pytest.mark.parametrize("signed", [True, False])
-def test_native_summaries_two_tiles_per_block(gpu_ctx, signed):
-    """Operands of at least 2048 tiles of 64 x 64 run the summary passes with
-    two tile rows per block, the second one's elements loaded into registers
-    while the first is summarized: 4100 x 2050 (65 x 33 tiles, an odd count
-    of tile rows, ragged last tiles) packed from a strided device source.
+@pytest.mark.parametrize("rows,cols", [(4100, 2050), (5130, 4110), (770, 65560)])
+def test_native_summaries_two_tiles_per_block(gpu_ctx, signed, rows, cols):
+    """Large operands from a strided device source. 4100 x 2050: one launch,
+    whose row waves and column blocks read their axes twice. 5130 x 4110: the
+    tile form with at least 2048 tiles of 64 x 64, two tile rows per block, the
+    second one's elements loaded into registers while the first is summarized
+    (81 x 65 tiles, an odd count of tile rows, ragged last tiles). 770 x 65560:
+    one launch with more than 65536 columns, so that column blocks stride.
     Values below 2^40 in magnitude keep the expected summaries exact in int64
     (numpy); the full-range 128-bit sums are checked on the smaller shapes."""
-    rows, cols = 4100, 2050
     rng = np.random.default_rng(77 + signed)
     lo, hi = (-(1 << 40) + 1, (1 << 40) - 1) if signed else (0, (1 << 40) - 1)
     x = rng.integers(lo, hi, size=(rows, cols), dtype=np.int64, endpoint=True)
     # extremes at tile boundaries and in the last, ragged tiles
-    x[0, 0], x[63, 64], x[64, 63], x[-1, -1], x[4096, 2048] = lo, hi, lo, hi, lo
+    x[0, 0], x[63, 64], x[64, 63], x[-1, -1], x[-3, -2] = lo, hi, lo, hi, lo
     M = _matrix(gpu_ctx, signed, rows, cols, 20)
     assert _pack(gpu_ctx, M, x if signed else x.astype(np.uint64), signed, True, ld=cols + 3) == r.SUCCESS
     bound, kind, R, C = M.exact_proof(gpu_ctx)
@@ -161,9 +164,9 @@ def _numpy_summaries(x, axis):
 
 @pytest.mark.parametrize("signed", [True, False])
 def test_proof_launches_past_one_grid(gpu_ctx, signed):
-    """Launch shapes whose grids stride: the finishing launch over more than
-    131072 axes (a 140000 x 8 operand, whose 2188 tile rows also run two per
-    block), and the product summaries over more than 32768 rows (a 33000 x 2
+    """Launch shapes whose grids stride: the tile form's finishing launch over
+    more than 131072 axes (a 140000 x 8 operand, whose 2188 tile rows also run
+    two per block), and the product summaries over more than 32768 rows (a 33000 x 2
     result, against the oracle's cell bounds)."""
     ctx = gpu_ctx
     lo, hi = (-(1 << 30) + 1, (1 << 30) - 1) if signed else (0, (1 << 30) - 1)
