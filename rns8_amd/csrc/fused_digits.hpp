@@ -338,10 +338,10 @@ bool fused_digits_shape(int64_t m, int64_t n, int64_t k, uint32_t nplanes, Fused
   // Whole calls, m x n x k, residue form / this form in us:
   //   planes >= 2 groups + 1: 8192 x 1 x 8192, 9 planes 147 / 106, n = 7 148 /
   //     134; 2000 x 7 x 1000, 9 planes 50 / 22; 128 x 7 x 256, 9 planes 18.8 /
-  //     17.3; 128 x 4 x 8192, 20 planes 111 / 30. Up to 4 planes this form's
+  //     17.3; 200 x 4 x 20000, 20 planes 135 / 50. Up to 4 planes this form's
   //     three launches cost more than they save (8000 x 5 x 300, 3 planes 12.8
-  //     / 15.3); at 5 and 6 only below 2^18 elements of A (128 x 5 x 256,
-  //     6 planes 13.9 / 14.3; 512 x 3 x 512, 5 planes 19.1 / 13.3).
+  //     / 15.3); at 5 and 6 also below 2^18 elements of A (128 x 5 x 256,
+  //     6 planes 13.9 / 14.3; but 512 x 3 x 512, 5 planes 19.1 / 13.3).
   //     Above 2^23 elements five planes' arithmetic hides behind the residue
   //     form's loads (5748 x 5 x 6620, 5 planes 79 / 89).
   //   3 groups <= 2 planes: while A is small enough to leave the residue form
@@ -349,6 +349,14 @@ bool fused_digits_shape(int64_t m, int64_t n, int64_t k, uint32_t nplanes, Fused
   //     planes 50 / 29; 2000 x 8 x 1000, 5 planes 33 / 21; but 8000 x 8 x 300,
   //     5 planes 16.6 / 17.7, 8192 x 8 x 8192, 9 planes 148 / 151, 512 x 8 x
   //     16000, 9 planes 57 / 61).
+  //     Deep and large ones of five and six planes lose (1160 x 10 x 6968, 6
+  //     planes 44.4 / 50.8; but 120 x 8 x 7040 45 / 28, 5041 x 7 x 1192 34 / 21).
+  //   The smallest products: the residue form of at most nine planes needs no
+  //     more than two launches up to 128 elements of K, this one three, so a pass
+  //     of product and export is bound by the launches (1000 x 1 x 64, 7 planes
+  //     14.3 / 16.0; 16 x 1 x 8, 9 planes 14.7 / 15.4; 4096 x 4 x 128, 9 planes
+  //     16.4 / 16.8; but 4096 x 2 x 100, 9 planes 16.2 / 15.8, 30000 x 1 x 64, 7
+  //     planes 17.5 / 15.6, 128 x 3 x 200, 8 planes 19.3 / 16.4).
   // The weights are 16 groups / m of A's bytes: with few rows per group
   // writing them costs more than it saves (9 planes: 32 x 2 x 100000 61 / 64,
   // 16 x 4 x 100000 60 / 98; 64 x 2 x 8000 53 / 17, 16 x 1 x 100000 60 / 43).
@@ -356,9 +364,31 @@ bool fused_digits_shape(int64_t m, int64_t n, int64_t k, uint32_t nplanes, Fused
   if (m < 16 * (2 * groups - 1) || groups > kMaxGroups || nplanes < 5) return false;
   const bool few = nplanes >= 2 * groups + 1 &&
                    (nplanes >= 7 || (work >= (int64_t{1} << 18) && work <= (int64_t{1} << 23)));
-  const bool mid = 3 * groups <= 2 * nplanes && k >= 512 && k <= 8192 && work >= (int64_t{1} << 18) &&
-                   work <= (int64_t{1} << 23);
+  const bool mid = 3 * groups <= 2 * nplanes && k >= 512 && work >= (int64_t{1} << 18) && work <= (int64_t{1} << 23) &&
+                   k <= (nplanes < 7 && work > (int64_t{1} << 22) ? 4096 : 8192);
   if (!few && !mid) return false;
+  if (k <= 128 && m <= 16384 && (nplanes <= 8 || (nplanes == 9 && (groups >= 3 || k <= 32)))) return false;
+  // Deeper products: the weights take 0.17 us per group and 1000 elements of K,
+  // whatever m, so the residue form is the faster one of few rows (128 x 7 x
+  // 200000, 9 planes 114 / 293; 128 x 4 x 65536, 9 planes 66 / 70; 800 x 7 x 32768,
+  // 9 planes 87 / 104; 16 x 1 x 560000, 7 planes 109 / 134) and this one of many
+  // (1200 x 4 x 65536, 9 planes 226 / 166; 512 x 2 x 100000, 9 planes 164 / 123;
+  // 200 x 4 x 65536, 20 planes 145 / 90). Both sides' times, in ns: this form's
+  // start, weights and read of A; the residue form's arithmetic over whole
+  // workgroups of 64 rows, at least its latency, per launch of up to 18 planes.
+  // Below three planes per group the weights count 15% more. Of 506 products
+  // from 16384 to 600000 deep, 9 run in this form and would be 1 to 10% faster in
+  // the other, 20 run in the other and would be 3 to 30% faster in this one.
+  if (k > 16384) {
+    if (nplanes < 7 && groups > 1) return false;
+    const int64_t launches = nplanes <= 18 ? 1 : 2, planes = (nplanes + launches - 1) / launches;
+    const double kd = static_cast<double>(k), md = static_cast<double>(m);
+    const double weights = 12000.0 + 0.17 * static_cast<double>(groups) * kd + md * kd / 690.0;
+    const double rows = static_cast<double>((m + 63) / 64 * 64);
+    const double residues = static_cast<double>(launches) *
+                            std::max(rows * kd * static_cast<double>(planes) / 3300.0, 10000.0 + 4200.0 * static_cast<double>(planes));
+    if ((nplanes < 3 * groups ? 1.15 : 1.0) * weights >= residues) return false;
+  }
   const Parts p = split(m, n, k, nplanes);
   out = FusedShape{};
   out.slices = static_cast<uint32_t>(p.slices);

@@ -1,0 +1,62 @@
+"""Which form of the fused native GEMM a product runs (CPU): the dispatch rules
+of fused.hip, fused_skinny.hip and fused_digits.hpp, asked of the library's own
+objects through tests/fused_forms_check.cpp. The digit form is expected where
+it measured faster and the residue form where that did."""
+from __future__ import annotations
+
+import shutil
+import subprocess
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parent.parent
+CSRC = ROOT / "rns8_amd" / "csrc"
+OBJS = [ROOT / "rns8_amd" / "_build" / f"{p.stem}.o" for p in sorted([*CSRC.glob("*.hip"), *CSRC.glob("*.cpp")])]
+
+
+@pytest.fixture(scope="module")
+def forms(tmp_path_factory):
+    gxx = shutil.which("g++")
+    if gxx is None:
+        pytest.skip("g++ not available")
+    if not all(p.is_file() for p in OBJS):
+        pytest.skip("library objects missing: run __graft_entry__.build()")
+    exe = tmp_path_factory.mktemp("forms") / "fused_forms_check"
+    subprocess.run([gxx, "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-isystem", "/opt/rocm/include", "-I",
+                    str(CSRC), "-I", str(ROOT / "include"), str(ROOT / "tests" / "fused_forms_check.cpp"),
+                    *map(str, OBJS), "-L/opt/rocm/lib", "-Wl,-rpath,/opt/rocm/lib", "-lamdhip64", "-pthread", "-o",
+                    str(exe)], check=True)
+
+    def ask(shapes):
+        text = "\n".join(" ".join(map(str, s)) for s in shapes) + "\n"
+        res = subprocess.run([str(exe)], input=text, capture_output=True, text=True, timeout=60, check=True)
+        return [line.split() for line in res.stdout.splitlines()]
+
+    return ask
+
+
+# (m, n, k, planes)
+RESIDUE_FASTER = [
+    # small products, bound by their launches
+    (16, 1, 8, 9), (16, 1, 100, 7), (1000, 1, 64, 7), (1000, 2, 100, 8), (128, 1, 100, 7), (4096, 4, 128, 9),
+    # deep ones of few rows, where writing the weights costs more than the residues
+    (128, 7, 200000, 9), (128, 4, 65536, 9), (800, 7, 32768, 9), (16, 1, 560000, 7), (952, 6, 103079, 7),
+    (52, 6, 130359, 5), (115, 5, 440956, 7), (64, 2, 560000, 9), (200, 7, 65536, 9),
+    # five and six planes
+    (1160, 10, 6968, 6), (5748, 5, 6620, 5), (53, 5, 53387, 6),
+    # many groups for the planes
+    (8192, 8, 8192, 9), (200, 16, 3000, 18),
+]
+DIGITS_FASTER = [
+    (8192, 1, 8192, 9), (8192, 7, 8192, 9), (2000, 7, 1000, 9), (128, 7, 256, 9), (200, 4, 20000, 20), (512, 3, 512, 5),
+    (2000, 9, 1000, 9), (64, 2, 8000, 9), (16, 1, 100000, 9), (30000, 1, 64, 7), (200000, 1, 8, 9), (128, 3, 200, 8),
+    (1200, 4, 65536, 9), (512, 2, 100000, 9), (200, 4, 65536, 20), (16, 1, 560000, 16), (5041, 7, 1192, 6),
+]
+
+
+def test_forms_taken_are_the_faster_ones(forms):
+    got = [f[0] for f in forms(RESIDUE_FASTER)]
+    assert got == ["residue"] * len(RESIDUE_FASTER), [s for s, g in zip(RESIDUE_FASTER, got) if g != "residue"]
+    got = [f[0] for f in forms(DIGITS_FASTER)]
+    assert got == ["digits"] * len(DIGITS_FASTER), [s for s, g in zip(DIGITS_FASTER, got) if g != "digits"]
