@@ -10,6 +10,9 @@ from pathlib import Path
 
 import pytest
 
+import test_gpu_fused_digits as digits
+import test_gpu_fused_skinny as skinny
+
 ROOT = Path(__file__).resolve().parent.parent
 CSRC = ROOT / "rns8_amd" / "csrc"
 OBJS = [ROOT / "rns8_amd" / "_build" / f"{p.stem}.o" for p in sorted([*CSRC.glob("*.hip"), *CSRC.glob("*.cpp")])]
@@ -60,3 +63,26 @@ def test_forms_taken_are_the_faster_ones(forms):
     assert got == ["residue"] * len(RESIDUE_FASTER), [s for s, g in zip(RESIDUE_FASTER, got) if g != "residue"]
     got = [f[0] for f in forms(DIGITS_FASTER)]
     assert got == ["digits"] * len(DIGITS_FASTER), [s for s, g in zip(DIGITS_FASTER, got) if g != "digits"]
+
+
+def test_gpu_tests_run_the_forms_they_are_for(forms):
+    assert [f[0] for f in forms([s[:4] for s in digits.SHAPES + digits.PARTS])] == ["digits"] * len(
+        digits.SHAPES + digits.PARTS)
+    assert [f[0] for f in forms([c[:4] for c in skinny.CASES])] == skinny.FORMS
+    assert [f[0] for f in forms([e[:4] for e in skinny.EXTENTS])] == [e[4] for e in skinny.EXTENTS]
+
+
+def test_gpu_test_shapes_run_in_parts(forms):
+    """The workspace holds at most 64 MiB of weights and of residues at once
+    (plus one slice's, one row group's, rounding): these products have more of
+    either, so they run in parts of it."""
+    limit = 64 << 20
+    (wm, wn, wk, wp, _), (rm, rn, rk, rp, _) = digits.PARTS
+    (_, w_slices, w_ks, w_bytes), (_, r_slices, _, r_bytes) = forms([digits.PARTS[0][:4], digits.PARTS[1][:4]])
+    groups = -(-wn * wp // 16)
+    all_weights = int(w_slices) * int(w_ks) // 16 * 2048 * groups
+    residues = int(w_slices) * 16 * groups * wm
+    assert all_weights > limit and int(w_bytes) < all_weights + residues
+    groups = -(-rn * rp // 16)
+    all_residues = int(r_slices) * 16 * groups * rm
+    assert all_residues > limit and int(r_bytes) < all_residues

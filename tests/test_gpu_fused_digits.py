@@ -1,8 +1,11 @@
 """The digit form of the fused native GEMM (results at most 16 columns wide
 whose planes x columns fill few 16-column groups): every group count, row
 counts around a wave's 32 and a workgroup's 128, K around a step of 16
-elements, a slice and the weights' parts, odd K and strides, int64 and uint64
-over the full range with the extremes placed. Planes against the oracle."""
+elements and a slice, more slices than the workspace holds weights for at
+once, more rows than it holds residues for, odd K and strides, int64 and uint64
+over the full range with the extremes placed. Planes against the oracle.
+tests/test_fused_forms.py checks on the CPU that every shape runs this form
+and that the two last ones run in parts."""
 from __future__ import annotations
 
 import ctypes
@@ -17,15 +20,19 @@ from rns8_amd import hip, inputs
 pytestmark = pytest.mark.gpu
 
 
+# (m, n, k, planes, elements of a row of A past k)
+SHAPES = [
+    (16, 1, 1, 16, 1), (31, 1, 15, 10, 1), (33, 1, 17, 16, 1), (127, 2, 31, 10, 3), (129, 3, 255, 9, 1),
+    (128, 5, 257, 9, 1), (112, 6, 511, 9, 1), (257, 4, 1040, 20, 0), (160, 7, 300, 9, 2), (140, 2, 4099, 5, 1),
+    (520, 8, 520, 9, 0), (513, 9, 513, 9, 1), (300, 8, 1000, 6, 0), (144, 4, 272, 20, 0), (20000, 1, 3, 7, 1),
+]
+# the weights of 560000 elements in two parts of the slices; 839000 rows'
+# residues of five groups in two parts of the rows
+PARTS = [(16, 1, 560000, 16, 2), (839000, 4, 8, 20, 0)]
+
+
 @pytest.mark.parametrize("signed", [True, False])
-@pytest.mark.parametrize(
-    "m,n,k,prefix,lda_extra",
-    [
-        (16, 1, 1, 7, 1), (31, 1, 15, 9, 1), (33, 1, 17, 16, 1), (127, 2, 31, 9, 3), (129, 3, 255, 9, 1),
-        (128, 5, 257, 9, 1), (112, 6, 511, 9, 1), (257, 4, 1040, 20, 0), (160, 7, 300, 8, 2), (140, 2, 4099, 5, 1),
-        (520, 8, 520, 9, 0), (513, 9, 513, 9, 1), (300, 16, 1000, 6, 0), (96, 4, 272, 20, 0),
-    ],
-)
+@pytest.mark.parametrize("m,n,k,prefix,lda_extra", SHAPES + PARTS)
 def test_fused_digits_planes(gpu_ctx, signed, m, n, k, prefix, lda_extra):
     ctx = gpu_ctx
     lda, ldb = k + lda_extra, n + 1

@@ -1,7 +1,8 @@
-"""GPU parity for the fused native-input GEMM's skinny form (results at most
-16 columns wide, fused_skinny.hip): C's residue planes from native device
-operands must equal, byte for byte, the planes rns8_gemm_rns computes from
-packed operands, and export to the exact product.
+"""GPU parity for the fused native-input GEMM on results at most 16 columns
+wide, in both of its forms (fused_skinny.hip's residues, fused_digits.hpp's
+digits): C's residue planes from native device operands must equal, byte for
+byte, the planes rns8_gemm_rns computes from packed operands, and export to the
+exact product.
 
 Cases cover one to 16 columns; 1 to 20 planes (one launch of up to 18
 planes, or two launches over the same rows); K below one 64-K
@@ -78,16 +79,24 @@ def _packed(ctx, plan, sem, bk, A, B, lda, ldb, signed):
 
 # (m, n, k, prefix, lda_extra, ldb_extra, signed, b_offset); A's stride is even
 CASES = [
-    (1000, 1, 8192, 9, 0, 0, True, 0),       # GEMV, one launch of nine planes, K split
+    (1000, 1, 8192, 9, 0, 0, True, 0),       # GEMV
     (1000, 3, 3001, 9, 3, 1, True, 8),       # odd K, strides above the width, B 8-byte aligned
     (33, 16, 70001, 5, 1, 0, False, 0),      # 16 columns, K above 65536
     (16, 8, 200000, 9, 0, 5, True, 0),       # one row block, many slices
     (7, 2, 40, 3, 2, 0, False, 0),           # K below one step, rows below one block
     (100, 5, 999, 20, 3, 0, True, 0),        # 20 planes: two launches of 10
     (50, 16, 5000, 10, 0, 0, False, 0),      # 10 planes in one launch
-    (200, 2, 3000, 18, 0, 0, True, 0),       # 18 planes in one launch (the largest group)
+    (200, 2, 3000, 18, 0, 0, True, 0),       # 18 planes in two groups of digits
     (300, 4, 1, 1, 1, 3, True, 8),           # K = 1, one plane (m = 256)
+    (200, 16, 3000, 18, 0, 0, True, 0),      # 18 planes in one launch of residues (its largest group)
+    (1000, 16, 8192, 9, 0, 0, True, 0),      # nine planes, K split in eight slices
+    (1000, 16, 3001, 9, 3, 1, False, 8),     # odd K, strides above the width, B 8-byte aligned
 ]
+# the form each of them runs (checked on the CPU by tests/test_fused_forms.py)
+FORMS = ["digits", "digits", "residue", "residue", "residue", "residue", "residue", "digits", "residue", "residue",
+         "residue", "residue"]
+# (m, n, k, prefix) of operands that end at their last logical element, and the form
+EXTENTS = [(70, 3, 3002, 9, "digits"), (70, 8, 3002, 7, "residue"), (16, 8, 3002, 9, "residue")]
 
 
 @pytest.mark.parametrize("case", range(len(CASES)))
@@ -109,13 +118,13 @@ def test_fused_skinny_planes_equal_packed_gemm(gpu_ctx, case):
 
 
 @pytest.mark.parametrize("signed", [True, False])
-def test_fused_skinny_reads_stay_in_logical_extent(gpu_ctx, signed):
+@pytest.mark.parametrize("m,n,k,prefix,form", EXTENTS)
+def test_fused_skinny_reads_stay_in_logical_extent(gpu_ctx, signed, m, n, k, prefix, form):
     """A in a buffer of exactly (m - 1) * lda + k elements and B of (k - 1) *
     ldb + n, each at the very end of a 64 KiB-aligned allocation: no load
     reaches past the last logical element, and the planes equal the packed
     GEMM's."""
-    m, n, k, prefix = 70, 3, 3002, 9  # A's start stays 16-byte aligned: (m - 1) * lda + k is even
-    lda, ldb = k + 30, n + 5
+    lda, ldb = k + 30, n + 5  # A's start stays 16-byte aligned: (m - 1) * lda + k is even
     A, B = _operands(1400 + signed, m, n, k, lda, ldb, signed)
     plan, sem, bk = _plan(gpu_ctx, signed, m, n, k, prefix, 2)
     a_elems, b_elems = (m - 1) * lda + k, (k - 1) * ldb + n
