@@ -207,6 +207,7 @@ __global__ __launch_bounds__(C::kThreads, kMinBlocks) void plane_gemm_kernel(Gem
   }
   u_first = __builtin_amdgcn_readfirstlane(u_first);
   u_end = __builtin_amdgcn_readfirstlane(u_end);
+  if (u_first >= u_end) return;  // (before any unit is decoded: a list ends with its last unit)
 
   // Units are decoded on the scalar unit (every value here is uniform) with
   // the host's reciprocals.
@@ -525,7 +526,6 @@ __global__ __launch_bounds__(C::kThreads, kMinBlocks) void plane_gemm_kernel(Gem
   // vmcnt waits below are what orders them. They are spread over the step (A
   // DMAs in the first half, B DMAs in the second): each one holds the texture
   // path for a while, and bunching a step's DMAs stalls MFMA issue.
-  if (u_first >= u_end) return;
   constexpr int kDmaStep = C::kDmaA + C::kDmaB;
   Frags f0, f1;
   uint32_t slot0 = 0, slot1 = C::kBufA, slot2 = 2 * C::kBufA;  // chunks c, c+1, c+2 of the compute position
@@ -794,10 +794,7 @@ hipError_t launch_gemm_cfg(const GemmArgs& args, int64_t k_slice, const PlaneCon
     map.k_begin = static_cast<uint32_t>(kb);
     map.k_stop = static_cast<uint32_t>(kstop);
     map.k_slice = static_cast<uint32_t>(ks);
-    // persistent grid: one workgroup per resident slot, a multiple of 8 (one
-    // share per XCD) when there are at least 8 units
-    uint64_t grid = units < slots ? units : slots;
-    if (grid >= 8) grid -= grid % 8;
+    const uint64_t grid = persistent_grid(units, slots);
     map.pairs = k_pairs(ks);
     hipLaunchKernelGGL((plane_gemm_kernel<Cf, kMinBlocks, false, kGrouped>), dim3(static_cast<unsigned>(grid)),
                        dim3(Cf::kThreads), 0, stream, args, consts, map, accumulate, tab);
@@ -848,8 +845,7 @@ template <typename Cf, int kMinBlocks>
 hipError_t launch_listed(const GemmArgs& args, const PlaneConsts& consts, const uint32_t* d_units, uint32_t units,
                          hipStream_t stream) {
   const uint64_t slots = static_cast<uint64_t>(device_cu_count()) * kMinBlocks;
-  uint64_t grid = units < slots ? units : slots;
-  if (grid >= 8) grid -= grid % 8;
+  const uint64_t grid = persistent_grid(units, slots);
   for (int64_t kb = 0; kb < args.k; kb += kSafeKBlock) {
     const int64_t kstop = min(args.k, kb + kSafeKBlock);
     UnitMap map{};

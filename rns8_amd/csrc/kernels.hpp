@@ -197,6 +197,18 @@ struct GemmShape {
   int64_t k_slice;    // K of one slice
   uint64_t ws_bytes;  // workspace: slices * nplanes * m * padded_ld(n) bytes when split, else 0
 };
+// Workgroups of a persistent launch: one per unit, at most one per resident
+// slot (a multiple of 8), and from 8 units on a multiple of 8, one share per
+// XCD. Rounded up: the XCDs' shares differ by one unit at most, so no workgroup
+// has more than one unit below `slots` units, and up to seven have none.
+// (Rounded down, up to seven units ran as a second round: 1786 x 1250 x 2044 at
+// 7 planes, 245 units of 256x256, 51.7 us; a 97 x 338 x 1058 plane, 12 units of
+// 64x64, 10.5 us.)
+inline uint64_t persistent_grid(uint64_t units, uint64_t slots) {
+  if (units < 8) return units;
+  const uint64_t shares = (units + 7) / 8 * 8, most = slots / 8 * 8;
+  return shares < most ? shares : most;
+}
 GemmShape choose_gemm_shape(int64_t m, int64_t n, int64_t k, uint32_t nplanes);
 // The skinny kernel's shape for n <= 16 (false for wider results), and its
 // launcher (skinny.hip): B and C rows of 16 bytes, args.slices ==

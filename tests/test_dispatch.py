@@ -1,7 +1,8 @@
-"""Which form of the fused native GEMM a product runs (CPU): the dispatch rules
-of fused.hip, fused_skinny.hip and fused_digits.hpp, asked of the library's own
-objects through tests/fused_forms_check.cpp. The digit form is expected where
-it measured faster and the residue form where that did."""
+"""Dispatch rules asked of the library's own objects (CPU), through
+tests/dispatch_check.cpp: which form of the fused native GEMM a product runs
+(fused.hip, fused_skinny.hip, fused_digits.hpp; the digit form is expected where
+it measured faster and the residue form where that did), and the plane GEMM's
+persistent grid."""
 from __future__ import annotations
 
 import shutil
@@ -19,24 +20,29 @@ OBJS = [ROOT / "rns8_amd" / "_build" / f"{p.stem}.o" for p in sorted([*CSRC.glob
 
 
 @pytest.fixture(scope="module")
-def forms(tmp_path_factory):
+def ask(tmp_path_factory):
     gxx = shutil.which("g++")
     if gxx is None:
         pytest.skip("g++ not available")
     if not all(p.is_file() for p in OBJS):
         pytest.skip("library objects missing: run __graft_entry__.build()")
-    exe = tmp_path_factory.mktemp("forms") / "fused_forms_check"
+    exe = tmp_path_factory.mktemp("dispatch") / "dispatch_check"
     subprocess.run([gxx, "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-isystem", "/opt/rocm/include", "-I",
-                    str(CSRC), "-I", str(ROOT / "include"), str(ROOT / "tests" / "fused_forms_check.cpp"),
+                    str(CSRC), "-I", str(ROOT / "include"), str(ROOT / "tests" / "dispatch_check.cpp"),
                     *map(str, OBJS), "-L/opt/rocm/lib", "-Wl,-rpath,/opt/rocm/lib", "-lamdhip64", "-pthread", "-o",
                     str(exe)], check=True)
 
-    def ask(shapes):
-        text = "\n".join(" ".join(map(str, s)) for s in shapes) + "\n"
+    def run(what, cases):
+        text = "\n".join(" ".join([what, *map(str, c)]) for c in cases) + "\n"
         res = subprocess.run([str(exe)], input=text, capture_output=True, text=True, timeout=60, check=True)
         return [line.split() for line in res.stdout.splitlines()]
 
-    return ask
+    return run
+
+
+@pytest.fixture(scope="module")
+def forms(ask):
+    return lambda shapes: ask("fused", shapes)
 
 
 # (m, n, k, planes)
@@ -86,3 +92,26 @@ def test_gpu_test_shapes_run_in_parts(forms):
     groups = -(-rn * rp // 16)
     all_residues = int(r_slices) * 16 * groups * rm
     assert all_residues > limit and int(r_bytes) < all_residues
+
+
+@pytest.mark.parametrize("slots", [256, 512, 1024])
+def test_persistent_grid_runs_every_unit_once(ask, slots):
+    """The plane GEMM's unit walk (gemm.hip: XCD x owns units [x units / 8, (x +
+    1) units / 8), its workgroups in lock step; grids that are no multiple of 8
+    walk all units) reaches every unit once, and no workgroup has a second unit
+    while a slot is free."""
+    counts = [*range(1, slots + 40), 3 * slots - 1, 3 * slots, 3 * slots + 9]
+    for units, (grid,) in zip(counts, ask("grid", [(u, slots) for u in counts])):
+        grid = int(grid)
+        assert 0 < grid <= slots
+        seen, most = [], 0
+        for b in range(grid):
+            if grid % 8 == 0:
+                x = b & 7
+                mine = list(range(x * units // 8 + (b >> 3), (x + 1) * units // 8, grid >> 3))
+            else:
+                mine = list(range(b, units, grid))
+            seen += mine
+            most = max(most, len(mine))
+        assert sorted(seen) == list(range(units)), units
+        assert most == -(-units // slots), (units, grid)

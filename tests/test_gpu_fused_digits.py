@@ -4,7 +4,7 @@ counts around a wave's 32 and a workgroup's 128, K around a step of 16
 elements and a slice, more slices than the workspace holds weights for at
 once, more rows than it holds residues for, odd K and strides, int64 and uint64
 over the full range with the extremes placed. Planes against the oracle.
-tests/test_fused_forms.py checks on the CPU that every shape runs this form
+tests/test_dispatch.py checks on the CPU that every shape runs this form
 and that the two last ones run in parts."""
 from __future__ import annotations
 

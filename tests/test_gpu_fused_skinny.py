@@ -92,7 +92,7 @@ CASES = [
     (1000, 16, 8192, 9, 0, 0, True, 0),      # nine planes, K split in eight slices
     (1000, 16, 3001, 9, 3, 1, False, 8),     # odd K, strides above the width, B 8-byte aligned
 ]
-# the form each of them runs (checked on the CPU by tests/test_fused_forms.py)
+# the form each of them runs (checked on the CPU by tests/test_dispatch.py)
 FORMS = ["digits", "digits", "residue", "residue", "residue", "residue", "residue", "digits", "residue", "residue",
          "residue", "residue"]
 # (m, n, k, prefix) of operands that end at their last logical element, and the form
