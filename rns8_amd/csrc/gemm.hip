@@ -149,7 +149,7 @@ struct UnitMap {
   DivU31 rows;    // kGroupM: tile rows of a full group
   DivU31 tail;    // tile rows of the last group (tiles_m - its first row)
   uint32_t k_begin, k_stop, k_slice;
-  uint32_t pairs;  // K chunks (two steps) every unit runs, at least 2; past the slice's K they read zeros
+  uint32_t pairs;  // K chunks (two steps) every unit runs; past the slice's K they read zeros
   // listed launches: two words per unit, (plane << 24 | tile row) and
   // (quadrant mask << 24 | tile column), in place of the arithmetic order
   const uint32_t* list;
@@ -306,7 +306,7 @@ __global__ __launch_bounds__(C::kThreads, kMinBlocks) void plane_gemm_kernel(Gem
   // are empty (every lane reads zero), which keeps the per-step DMA count and
   // therefore the vmcnt bookkeeping uniform. The cursor steps by additions
   // and enters the next unit exactly when the compute position is two chunks
-  // from the end of its own: one wave per SIMD issues every instruction, and
+  // from the end of its own (units of one chunk: at each, the unit after the next): one wave per SIMD issues every instruction, and
   // the ~45 scalar ones of decoding a unit and rebuilding its resources at
   // every step left the matrix cores idle meanwhile.
   struct Cursor {
@@ -530,6 +530,9 @@ __global__ __launch_bounds__(C::kThreads, kMinBlocks) void plane_gemm_kernel(Gem
   Frags f0, f1;
   uint32_t slot0 = 0, slot1 = C::kBufA, slot2 = 2 * C::kBufA;  // chunks c, c+1, c+2 of the compute position
   uint32_t stage0 = 0, stage2 = 2 * C::kBufB;                  // B stages of the pair and of the next pair
+  // (units of one chunk: the second is the next unit's)
+  const bool one_chunk = map.pairs == 1u;
+  auto unit_cursor = [&](uint32_t u) { return cursor_of(decode(min(u, u_end - 1)), u < u_end); };
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
     const v4i sa = src_a();
@@ -542,6 +545,7 @@ __global__ __launch_bounds__(C::kThreads, kMinBlocks) void plane_gemm_kernel(Gem
       for (int i = 0; i < C::kDmaB; ++i) dma_b(sb, (2 * c + half) * C::kBufB, i);
     }
     cursor_advance();
+    if (c == 0 && one_chunk) cur = unit_cursor(u_first + u_step);
   }
   __builtin_amdgcn_s_waitcnt(wait_vm(2 * kDmaStep));  // chunk 0 landed
   __syncthreads();
@@ -597,10 +601,10 @@ __global__ __launch_bounds__(C::kThreads, kMinBlocks) void plane_gemm_kernel(Gem
   };
   for (uint32_t u = u_first; u < u_end; u += u_step) {
     const Unit U = decode(u);
-    const Cursor next = cursor_of(decode(min(u + u_step, u_end - 1)), u + u_step < u_end);
-    // The cursor enters the next unit by selects at the pair two chunks
-    // before the end (a branch there makes the compiler duplicate the pair
-    // and spill accumulators).
+    const Cursor next = unit_cursor(u + (one_chunk ? 2 * u_step : u_step));
+    // The cursor enters the next unit (of one-chunk units the one after it) by
+    // selects at the pair two chunks before the end (a branch there makes the
+    // compiler duplicate the pair and spill accumulators).
     auto enter_next = [&](bool enter) {
       cur.a = enter ? next.a : cur.a;
       cur.b = enter ? next.b : cur.b;
@@ -610,7 +614,7 @@ __global__ __launch_bounds__(C::kThreads, kMinBlocks) void plane_gemm_kernel(Gem
       cur.dec = enter ? next.dec : cur.dec;
     };
     uint32_t n = map.pairs;
-    enter_next(n == 2u);
+    enter_next(n <= 2u);
     pair(std::true_type{});
     for (--n; n; --n) {
       enter_next(n == 2u);
@@ -683,7 +687,7 @@ GemmTile choose_tile(int64_t m, int64_t n, int64_t k_slice, int64_t plane_slices
       {GemmTile::k128x256, 128, 256, 350, 84, 200},  {GemmTile::k128x128, 128, 128, 300, 45, 100},
       {GemmTile::k64x64, 64, 64, 250, 25, 60}};
   constexpr int64_t kCus = 256;
-  const int64_t chunks = std::max<int64_t>((std::min<int64_t>(k_slice, kSafeKBlock) + 127) / 128, 2);
+  const int64_t chunks = (std::min<int64_t>(k_slice, kSafeKBlock) + 127) / 128;
   GemmTile best = GemmTile::k128x128;
   double best_cost = 0;
   for (const TileCost& t : kCosts) {
@@ -756,9 +760,8 @@ int device_cu_count() {
   return cus;
 }
 
-// K chunks of 128 that every unit of a launch runs: at least the two whose
-// DMAs a unit's prologue issues.
-uint32_t k_pairs(int64_t k_slice) { return static_cast<uint32_t>(std::max<int64_t>((k_slice + 127) / 128, 2)); }
+// K chunks of 128 that every unit of a launch runs.
+uint32_t k_pairs(int64_t k_slice) { return static_cast<uint32_t>((k_slice + 127) / 128); }
 
 // Ungrouped launches pass a NoTaskTable and ntasks = 1; grouped ones the
 // task table and its task count (at most kMaxGroupTasks). `k_slice` is the

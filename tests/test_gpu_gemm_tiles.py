@@ -1,7 +1,7 @@
 """Every output tile of the plane GEMM (256x256, 256x128, 128x256, 128x128,
 64x64) at its edges: rows and columns one past and one short of a tile, K of
 one element, around the 64-deep step and the 128-deep A chunk, odd chunk
-counts, and tile counts that leave some workgroups of the grid without a tile. Finite products, compared with float64 matrix products on the CPU
+counts, several tiles of one chunk per workgroup, and tile counts that leave some workgroups of the grid without a tile. Finite products, compared with float64 matrix products on the CPU
 (k * 255^2 < 2^53: every sum is exact)."""
 from __future__ import annotations
 
@@ -20,9 +20,10 @@ pytestmark = pytest.mark.gpu
         ("64x64", 1, 17, 1), ("64x64", 63, 65, 63), ("64x64", 65, 64, 65), ("64x64", 130, 127, 127),
         ("64x64", 64, 191, 129), ("64x64", 200, 300, 1000), ("64x64", 190, 180, 70), ("64x64", 97, 338, 1058),
         ("128x128", 2049, 1030, 260), ("128x128", 2050, 1025, 385), ("128x128", 2709, 707, 20),
+        ("128x128", 4200, 4300, 100), ("128x128", 4200, 4300, 1),
         ("256x128", 1100, 4097, 1025), ("256x128", 1568, 2477, 1060),
         ("128x256", 2373, 3211, 1036),
-        ("256x256", 4097, 3000, 129), ("256x256", 3439, 3594, 20), ("256x256", 4095, 4090, 641), ("256x256", 4300, 3800, 200),
+        ("256x256", 4097, 3000, 129), ("256x256", 3439, 3594, 20), ("256x256", 4095, 4090, 641), ("256x256", 4300, 3800, 200), ("256x256", 5000, 9000, 65),
     ],
 )
 @pytest.mark.parametrize("modulus", [251, 256])
