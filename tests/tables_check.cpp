@@ -89,7 +89,7 @@ void fail(const char* what, uint32_t m, long long a, long long b, long long c) {
 uint32_t s_max_i32(const ModulusConsts& c) {
   uint32_t bytes = 0;
   for (int k = 0; k < 4; ++k) bytes += (c.pow_lo >> (8 * k)) & 0xFFu;
-  return 255u * bytes + c.off_i32;
+  return 255u * bytes + (c.off_i32 > c.off_acc ? c.off_i32 : c.off_acc);
 }
 
 void check_quot() {
@@ -140,11 +140,33 @@ void check_reduce32() {
   for (int i = 0; i < 40000; ++i) xs.push_back(static_cast<int32_t>(rng.next()));
   for (int i = 0; i < 20000; ++i) xs.push_back(static_cast<int32_t>(rng.next() % 2147483649ull) - (1 << 30));
   uint64_t checks = 0;
+  // The plane GEMM's and the digit form's sums: at most 65536 products of 2^14
+  // and a carried residue, around kGemmAccBias, which is 0 modulo 256 (a modulus
+  // of 256 takes the low byte of the biased sum).
+  constexpr int64_t kAccMax = (int64_t{1} << 30) + 128;
+  if (kGemmAccBias % 256 != 0 || kGemmAccBias < kAccMax || (int64_t{1} << 32) - kGemmAccBias <= kAccMax)
+    fail("accumulator bias", 0, kGemmAccBias, kAccMax, 0);
+  std::vector<int32_t> sums = {0, 1, -1, 127, -128, 128, -129, 65535, -65536, 1 << 30, -(1 << 30),
+                               static_cast<int32_t>(kAccMax), static_cast<int32_t>(-kAccMax)};
+  for (int i = 0; i < 40000; ++i) sums.push_back(static_cast<int32_t>(static_cast<int64_t>(rng.next() % (2 * kAccMax + 1)) - kAccMax));
   for (uint32_t m = 2; m <= 256; ++m) {
     const ModulusConsts c = make_modulus_consts(m);
-    // the epilogue's reduction: u = x + 2^31, s - H = dot(bytes(u), pow_lo)
-    // + (off_i32 - H)
-    if (c.off_i32 < c.half || c.off_i64 < c.half || c.off_u64 < c.half) fail("offset below H", m, c.off_i32, c.off_i64, c.off_u64);
+    // the finalizes' and the skinny kernels' reduction: u = x + 2^31, s - H =
+    // dot(bytes(u), pow_lo) + (off_i32 - H)
+    if (c.off_i32 < c.half || c.off_i64 < c.half || c.off_u64 < c.half || c.off_acc < c.half)
+      fail("offset below H", m, c.off_i32, c.off_i64, c.off_u64);
+    // the plane GEMM's epilogue: the same from u = x + kGemmAccBias and off_acc;
+    // the digit form's: s from both, its quotient by the 32-bit reciprocal
+    for (int32_t x : sums) {
+      const uint32_t u = static_cast<uint32_t>(x) + kGemmAccBias;
+      const int64_t want = centered_ref(x, m);
+      const uint32_t r = centered_byte(udot4(u, c.pow_lo, c.off_acc - c.half), c.q_shift, c.half << c.q_shift, c.q_recip, m);
+      if (static_cast<int8_t>(r) != want) fail("accumulator residue", m, x, static_cast<int8_t>(r), want);
+      const uint32_t s = udot4(u, c.pow_lo, c.off_acc);
+      const int8_t d = static_cast<int8_t>(s - umulhi(s, c.recip) * m - c.half);
+      if (d != want) fail("digit residue", m, x, d, want);
+      checks += 2;
+    }
     for (size_t i = 0; i + 4 <= xs.size(); i += 4) {
       uint32_t r[4];
       for (int e = 0; e < 4; ++e) {

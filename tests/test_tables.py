@@ -46,8 +46,8 @@ def test_quotients_exhaustive(checker):
 
 
 def test_epilogue_reduction_int32(checker):
-    """int32 sums (full range and the |x| <= 2^30 + 128 the GEMM produces) ->
-    packed centered int8, every modulus 2..256."""
+    """int32 sums (full range, and the |x| <= 2^30 + 128 the GEMM produces, from
+    its biased accumulators) -> packed centered int8, every modulus 2..256."""
     _run(checker, "reduce32")
 
 
