@@ -37,58 +37,23 @@ constexpr int kColsPerBlock = 8;           // 4 lanes of 2 columns; kThreads / 4
 constexpr int kRowLanes = kThreads / 4;
 constexpr int64_t kMaxBlocks = 8192;       // of either kind; larger operands stride
 
-// 96-bit sum of 64-bit values.
-struct Sum96 {
-  u64 lo = 0;
-  uint32_t hi = 0;
-  __device__ __forceinline__ void add(u64 x, uint32_t x_hi = 0) {
-    lo += x;
-    hi += x_hi + (lo < x ? 1u : 0u);
-  }
-  __device__ __forceinline__ u128 value() const { return (static_cast<u128>(hi) << 64) | lo; }
-};
-
-// One lane's running summary over biased values u (bias(): their unsigned
-// order is the order of x; at most 2^32 of them). The absolute sum comes from
-// the sum of the positive parts: sum |x| = 2 sum max(x, 0) - sum x.
-template <bool Signed>
-struct Extremes {
-  u64 hi = 0, lo = ~u64{0};
-  Sum96 sum, pos;
-  __device__ __forceinline__ void add(u64 u) {
-    hi = u > hi ? u : hi;
-    lo = u < lo ? u : lo;
-    sum.add(u);
-    if constexpr (Signed) pos.add(static_cast<int64_t>(u) < 0 ? u & ~(u64{1} << 63) : 0);  // x = u - 2^63
-  }
-  // merges the lanes whose index differs in bits kFrom .. 32
-  template <int kFrom>
-  __device__ __forceinline__ void merge() {
+// Merges the lanes whose index differs in bits kFrom .. 32.
+template <int kFrom, bool Signed>
+__device__ __forceinline__ void merge_lanes(Extremes<Signed>& e) {
 #pragma unroll
-    for (int m = kFrom; m < 64; m <<= 1) {
-      const u64 h = __shfl_xor(hi, m), l = __shfl_xor(lo, m);
-      hi = h > hi ? h : hi;
-      lo = l < lo ? l : lo;
-      const u64 s = __shfl_xor(sum.lo, m);
-      sum.add(s, __shfl_xor(sum.hi, m));
-      if constexpr (Signed) {
-        const u64 q = __shfl_xor(pos.lo, m);
-        pos.add(q, __shfl_xor(pos.hi, m));
-      }
+  for (int m = kFrom; m < 64; m <<= 1) {
+    Extremes<Signed> o;
+    o.hi = __shfl_xor(e.hi, m);
+    o.lo = __shfl_xor(e.lo, m);
+    o.sum.lo = __shfl_xor(e.sum.lo, m);
+    o.sum.hi = __shfl_xor(e.sum.hi, m);
+    if constexpr (Signed) {
+      o.pos.lo = __shfl_xor(e.pos.lo, m);
+      o.pos.hi = __shfl_xor(e.pos.hi, m);
     }
+    e.merge(o);
   }
-  // of `count` values in all (this lane's are a part of them)
-  __device__ __forceinline__ AxisPartial partial(u64 count) const {
-    const u128 s = sum.value();
-    return AxisPartial{hi, ~lo, s, Signed ? 2 * pos.value() - (s - (static_cast<u128>(count) << 63)) : s};
-  }
-};
-// The sum of |x - c| over `count` values from sum max(x - c, 0) and the sum of
-// the biased values: 2 sum max(u - cu, 0) - (sum u - count cu).
-__device__ __forceinline__ u128 deviation_total(const Sum96& above, u128 sum, u64 count, u64 cu) {
-  return 2 * above.value() - (sum - static_cast<u128>(count) * cu);
 }
-__device__ __forceinline__ void add_above(Sum96& above, u64 u, u64 cu) { above.add(u > cu ? u - cu : 0); }
 template <int kFrom>
 __device__ __forceinline__ void merge_lanes(Sum96& s) {
 #pragma unroll
@@ -170,7 +135,7 @@ __global__ __launch_bounds__(kThreads, 4) void native_axes_kernel(const uint64_t
         fetch(c0);
         each(c0, [&](u64 u) { acc.add(u); });
       }
-      acc.template merge<1>();
+      merge_lanes<1>(acc);
       // the record is stored before the second pass and its deviation sum
       // after it: held meanwhile, its 32 registers would spill
       u64 cu;
@@ -275,7 +240,7 @@ __global__ __launch_bounds__(kThreads, 4) void native_axes_kernel(const uint64_t
     // the count enters once (wave 0's partial)
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
-      acc[e].template merge<4>();
+      merge_lanes<4>(acc[e]);
       if (lane < 4) part[wave][pair + e] = acc[e].partial(wave == 0 ? static_cast<u64>(rows) : 0);
     }
     __syncthreads();

@@ -231,8 +231,8 @@ RNS8_XA U256 cell_bound(const AxisTerms& a, const AxisTerms& b) {
 
 // ---- native summaries: what the pack-time passes compute ------------------
 
-// A partial summary of part of one axis (one 64 x 64 tile's share of a row
-// or a column), in "biased" values u (x + 2^63 for int64, x for uint64),
+// A partial summary of part of one axis (a wave's share of a column, one 64 x
+// 64 tile's of a row or a column), in "biased" values u (x + 2^63 for int64, x for uint64),
 // whose unsigned order is the order of x. Pass 1 fills every field; pass 2
 // keeps the sum of |x - centre| in `sum`. Partials of at most 2^63 values
 // are exact in these widths (sums below 2^127).
@@ -254,19 +254,59 @@ RNS8_XA u64 magnitude(u64 raw, bool is_signed) {
   return x < 0 ? u64{0} - raw : raw;  // |INT64_MIN| = 2^63 fits
 }
 RNS8_XA AxisPartial empty_partial() { return AxisPartial{0, 0, 0, 0}; }
-RNS8_XA void partial_add(AxisPartial& p, u64 raw, bool is_signed) {
-  const u64 u = bias(raw, is_signed);
-  p.hi = u > p.hi ? u : p.hi;
-  p.not_lo = ~u > p.not_lo ? ~u : p.not_lo;
-  p.sum += u;
-  p.abs_sum += magnitude(raw, is_signed);
-}
 RNS8_XA void partial_merge(AxisPartial& p, const AxisPartial& o) {
   p.hi = o.hi > p.hi ? o.hi : p.hi;
   p.not_lo = o.not_lo > p.not_lo ? o.not_lo : p.not_lo;
   p.sum += o.sum;
   p.abs_sum += o.abs_sum;
 }
+// ---- the one-launch form (exact_axes.hip native_axes_kernel) ----------------
+
+// 96-bit sum of 64-bit values.
+struct Sum96 {
+  u64 lo = 0;
+  uint32_t hi = 0;
+  RNS8_XA void add(u64 x, uint32_t x_hi = 0) {
+    lo += x;
+    hi += x_hi + (lo < x ? 1u : 0u);
+  }
+  RNS8_XA u128 value() const { return (static_cast<u128>(hi) << 64) | lo; }
+};
+
+// One lane's running summary over biased values u (bias(): their unsigned
+// order is the order of x; at most 2^32 of them). The absolute sum comes from
+// the sum of the positive parts: sum |x| = 2 sum max(x, 0) - sum x.
+template <bool Signed>
+struct Extremes {
+  u64 hi = 0, lo = ~u64{0};
+  Sum96 sum, pos;
+  RNS8_XA void add(u64 u) {
+    hi = u > hi ? u : hi;
+    lo = u < lo ? u : lo;
+    sum.add(u);
+    if constexpr (Signed) pos.add(static_cast<int64_t>(u) < 0 ? u & ~(u64{1} << 63) : 0);  // x = u - 2^63
+  }
+  RNS8_XA void merge(const Extremes& o) {
+    hi = o.hi > hi ? o.hi : hi;
+    lo = o.lo < lo ? o.lo : lo;
+    sum.add(o.sum.lo, o.sum.hi);
+    if constexpr (Signed) pos.add(o.pos.lo, o.pos.hi);
+  }
+  // of `count` values in all (this lane's are a part of them)
+  RNS8_XA AxisPartial partial(u64 count) const {
+    const u128 s = sum.value();
+    return AxisPartial{hi, ~lo, s, Signed ? 2 * pos.value() - (s - (static_cast<u128>(count) << 63)) : s};
+  }
+};
+// max(u - cu, 0), summed, and from that sum, the sum of |x - c| over `count`
+// values whose biased values sum to `sum`: 2 sum max(u - cu, 0) - (sum u - count cu).
+RNS8_XA void add_above(Sum96& above, u64 u, u64 cu) { above.add(u > cu ? u - cu : 0); }
+RNS8_XA u128 deviation_total(const Sum96& above, u128 sum, u64 count, u64 cu) {
+  return 2 * above.value() - (sum - static_cast<u128>(count) * cu);
+}
+
+// ---- the tile form (exact_axes.hip tiled_axes_pass, tiled_axes_finish) -------
+
 // The running partial of one lane over at most 2^32 values, with the sums
 // as a 64-bit word plus a count of carries out of it.
 struct PartialAcc {

@@ -19,13 +19,14 @@
 //     for 0 <= a, b < 2^256: sat_mul, sat_add, min and max.
 //
 //   native <S|U> <rows> <cols> then rows x cols values
-//     the summaries of a 64-bit operand, computed in the device passes'
-//     decomposition (per 64 x 64 tile partials of each row and column,
-//     extremes as maxima of biased values, merged per axis) with the same
+//     the summaries of a 64-bit operand, computed in both device forms'
+//     decompositions (per 64 x 64 tile partials of each row and column, merged
+//     per axis; and whole axes over a block's lanes and waves) with the same
 //     functions. Output: max |x|, then one line per row and per column with
-//     the seven fields above.
+//     the seven fields above, or a line saying where the two forms differ.
 #include <cstdint>
 #include <cstdio>
+#include <cstring>
 #include <iostream>
 #include <string>
 #include <vector>
@@ -154,11 +155,50 @@ int gemm_case() {
   return 0;
 }
 
-// The device passes' decomposition (exact_axes.hip native_axes_pass and
-// native_axes_finish): per 64 x 64 tile, each row's and each column's
+// The one-launch form's decomposition (exact_axes.hip native_axes_kernel): a
+// row is 64 lanes of neighbouring pairs, merged; a column is 8 waves of 16
+// lane classes, merged per wave and then as partials, the count entering once.
+template <bool Signed>
+AxisRecord one_launch_axis(const std::vector<u64>& raw, bool is_row) {
+  const std::size_t n = raw.size(), groups = is_row ? 1 : 8, lanes = is_row ? 64 : 16;
+  auto lane_of = [&](std::size_t j) { return is_row ? j / 2 % 64 : j % 16; };
+  auto group_of = [&](std::size_t j) { return is_row ? std::size_t{0} : j / 16 % 8; };
+  auto merged = [&](std::size_t g, auto make, auto add) {
+    std::vector<decltype(make())> part(lanes, make());
+    for (std::size_t j = 0; j < n; ++j)
+      if (group_of(j) == g) add(part[lane_of(j)], bias(raw[j], Signed));
+    return part;
+  };
+  AxisPartial p = empty_partial();
+  for (std::size_t g = 0; g < groups; ++g) {
+    auto part = merged(g, [] { return Extremes<Signed>{}; }, [](Extremes<Signed>& e, u64 u) { e.add(u); });
+    for (std::size_t m = 1; m < lanes; m <<= 1)  // the butterfly: lane l takes in lane l ^ m
+      for (std::size_t l = 0; l < lanes; ++l)
+        if (!(l & m)) {
+          const Extremes<Signed> a = part[l], b = part[l ^ m];
+          part[l].merge(b);
+          part[l ^ m].merge(a);
+        }
+    const AxisPartial q = part[0].partial(g == 0 ? n : 0);
+    if (g == 0) p = q;
+    else partial_merge(p, q);
+  }
+  AxisRecord rec = native_record(p, n, Signed);
+  const u64 cu = bias(static_cast<u64>(record_centre(rec)), Signed);
+  Sum96 above;
+  for (std::size_t g = 0; g < groups; ++g) {
+    auto part = merged(g, [] { return Sum96{}; }, [&](Sum96& s, u64 u) { add_above(s, u, cu); });
+    for (const Sum96& s : part) above.add(s.lo, s.hi);
+  }
+  put_u128(rec.deviation_sum, deviation_total(above, p.sum, n, cu));
+  return rec;
+}
+
+// The tile form's decomposition (exact_axes.hip tiled_axes_pass and
+// tiled_axes_finish): per 64 x 64 tile, each row's and each column's
 // partial over two halves of 32, merged; then each axis's partials merged in
 // tile order, the record built, and a second pass of deviation partials
-// around the records' centres.
+// around the records' centres. The records must equal the one-launch form's.
 int native_case() {
   std::string sem;
   int64_t rows, cols;
@@ -219,6 +259,17 @@ int native_case() {
         }
       }
   }
+  for (int by_row = 1; by_row >= 0; --by_row)
+    for (int64_t axis = 0; axis < (by_row ? rows : cols); ++axis) {
+      std::vector<u64> v;
+      for (int64_t j = 0; j < (by_row ? cols : rows); ++j) v.push_back(by_row ? xs[axis * cols + j] : xs[j * cols + axis]);
+      const AxisRecord one = sgn ? one_launch_axis<true>(v, by_row != 0) : one_launch_axis<false>(v, by_row != 0);
+      const AxisRecord& two = by_row ? rr[axis] : cr[axis];
+      if (std::memcmp(&one, &two, sizeof one) != 0) {
+        std::cout << "the forms differ at " << (by_row ? "row " : "column ") << axis << "\n";
+        return 1;
+      }
+    }
   u64 top = 0;
   for (const auto& r : rr) top = r.max_magnitude[0] > top ? r.max_magnitude[0] : top;
   std::cout << hex(from128(top)) << "\n";
@@ -247,7 +298,9 @@ int ops_case() {
 int main() {
   std::string tag;
   while (std::cin >> tag) {
-    if (tag == "native") native_case();
+    if (tag == "native") {
+      if (native_case()) return 1;
+    }
     else if (tag == "case") gemm_case();
     else if (tag == "ops") ops_case();
     else return 2;

@@ -201,13 +201,13 @@ def _axis_tuple(a: xr.Axis):
 
 
 @pytest.mark.parametrize("signed", [True, False])
-@pytest.mark.parametrize("rows,cols", [(1, 1), (1, 7), (9, 1), (13, 40), (67, 5), (70, 130), (129, 65)])
+@pytest.mark.parametrize("rows,cols", [(1, 1), (1, 7), (9, 1), (13, 40), (67, 5), (70, 130), (129, 65), (3, 300), (300, 2)])
 def test_native_summaries_match_unbounded(checker, signed, rows, cols):
-    """The summaries of a 64-bit operand, computed in the device passes'
-    decomposition (per-tile partials of each row and column, extremes as
-    maxima of biased values; more than one 64 x 64 tile in the larger cases),
-    equal the unbounded ones, with the int64 / uint64 extremes placed in
-    every case."""
+    """The summaries of a 64-bit operand, computed in both device forms'
+    decompositions (per-tile partials of each row and column, more than one 64 x
+    64 tile in the larger cases; whole axes over lanes and waves, the absolute
+    and deviation sums from positive parts in 96 bits), equal the unbounded
+    ones, with the int64 / uint64 extremes placed in every case."""
     rng = random.Random(rows * 1000 + cols + signed)
     lo, hi = (-(1 << 63), (1 << 63) - 1) if signed else (0, (1 << 64) - 1)
     x = _native(rng, rows, cols, lo, hi)
@@ -247,3 +247,17 @@ def test_saturating_word_arithmetic(checker):
     for (a, b), line in zip(pairs, res.stdout.split("\n")):
         got = [int(x, 16) for x in line.split()]
         assert got == [_sat(a * b), _sat(a + b), min(a, b), max(a, b)], (hex(a), hex(b))
+
+
+@pytest.mark.parametrize("signed", [True, False])
+@pytest.mark.parametrize("value", ["lo", "hi", "mixed"])
+def test_native_summaries_of_extremes(checker, signed, value):
+    """Axes of nothing but extremes: every addition carries out of 64 bits (or
+    none does), and the positive parts are all of the sum or none of it."""
+    lo, hi = (-(1 << 63), (1 << 63) - 1) if signed else (0, (1 << 64) - 1)
+    x = [[{"lo": lo, "hi": hi, "mixed": (lo, hi, hi - 1)[(3 * i + j) % 3]}[value] for j in range(70)] for i in range(140)]
+    maximum, got_rows, got_cols = _native_summaries(checker, signed, x)
+    want = xr.native_operand(x)
+    assert maximum == want.max_magnitude
+    assert got_rows == [_axis_tuple(a) for a in want.rows]
+    assert got_cols == [_axis_tuple(a) for a in want.cols]
