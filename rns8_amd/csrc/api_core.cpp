@@ -639,6 +639,9 @@ rns8_status rns8_get_device_info(rns8_context* ctx, rns8_device_info* out) {
   });
 }
 
+// The instruction of every plane GEMM kernel, the skinny one included.
+static constexpr char kIsaEvidence[] = "gfx950 v_mfma_i32_16x16x64_i8";
+
 rns8_status rns8_get_backend_capability_info(rns8_backend_kind backend, rns8_backend_capability_info* out) {
   return guard([&]() -> rns8_status {
     if (!out || !valid_abi(out->struct_size, out->abi_version, sizeof(*out))) return RNS8_INVALID_ARGUMENT;
@@ -659,12 +662,12 @@ rns8_status rns8_get_backend_capability_info(rns8_backend_kind backend, rns8_bac
     out->exact_differential_validated = ours ? 1u : 0u;
     copy_text(out->backend_name, sizeof(out->backend_name), ours ? "hip_direct_gfx950" : "not_in_this_library");
     copy_text(out->selected_kernel, sizeof(out->selected_kernel),
-              ours ? "plane_gemm_kernel<64> v_mfma_i32_32x32x32_i8" : "");
+              ours ? "plane_gemm_kernel v_mfma_i32_16x16x64_i8" : "");
     copy_text(out->library_name, sizeof(out->library_name), "rns8_mi355x");
     copy_text(out->library_version, sizeof(out->library_version), "0.1");
     copy_text(out->epilogue_mode, sizeof(out->epilogue_mode), ours ? "in_register_centered_reduction" : "");
     copy_text(out->workspace_mode, sizeof(out->workspace_mode), ours ? "resident_planes_splitk_int8_residues" : "");
-    copy_text(out->isa_evidence, sizeof(out->isa_evidence), ours ? "gfx950 v_mfma_i32_32x32x32_i8" : "");
+    copy_text(out->isa_evidence, sizeof(out->isa_evidence), ours ? kIsaEvidence : "");
     copy_text(out->status, sizeof(out->status), ours ? (hip ? "available" : "no_hip_device") : "unsupported_backend");
     copy_text(out->detail, sizeof(out->detail),
               ours ? "MI355X-native HIP_DIRECT implementation" : "backend not part of the MI355X library");
@@ -878,8 +881,7 @@ rns8_status rns8_get_plan_backend_info(const rns8_plan* plan, rns8_plan_backend_
     copy_text(out->epilogue_mode, sizeof(out->epilogue_mode), "in_register_centered_reduction");
     copy_text(out->workspace_mode, sizeof(out->workspace_mode),
               plan->splitk_slices > 1 ? "splitk_int8_residues" : "none");
-    copy_text(out->isa_evidence, sizeof(out->isa_evidence),
-              "gfx950 v_mfma_i32_16x16x64_i8");
+    copy_text(out->isa_evidence, sizeof(out->isa_evidence), kIsaEvidence);
     out->accumulator_k_block_size = static_cast<uint64_t>(plan->desc.k < kSafeKBlock ? plan->desc.k : kSafeKBlock);
     out->accumulator_k_block_cap = static_cast<uint64_t>(kSafeKBlock);
     out->accumulator_modulus = uses_finite_storage(plan->desc.semantics) ? plan->desc.finite_modulus : 0;

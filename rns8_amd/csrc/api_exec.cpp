@@ -169,7 +169,7 @@ rns8_status run_gemm_tiled(rns8_context& ctx, const rns8_plan& plan, const rns8_
   const uint32_t planes = storage_prefix(plan);
   const GemmArgs g = gemm_args(plan, A, B, C, nullptr, planes, 1);
   if (hipSetDevice(ctx.device_id) != hipSuccess) return RNS8_BACKEND_FAILURE;
-  hipError_t e = launch_gemm_listed(g, make_ladder_plane_consts(planes), plan.units, plan.unit_count,
+  hipError_t e = launch_gemm_listed(g, make_ladder_plane_consts(), plan.units, plan.unit_count,
                                     plan.unit_edge, stream);
   if (e == hipErrorInvalidValue) return RNS8_UNSUPPORTED_BACKEND;
   if (e == hipSuccess) e = launch_zero_tiles(C.planes, C.plane_ld, C.plane_pitch, plan.zero_fills,
@@ -195,7 +195,7 @@ rns8_status gemm_rns(rns8_context* ctx, const rns8_plan* plan, const rns8_matrix
   if (per_tile_kind(plan->desc.bound_kind) && !plan->schedule.entries.empty())
     st = run_gemm_tiled(*ctx, *plan, *A, *B, *C, stream);
   else
-    st = run_gemm(*ctx, *plan, *A, *B, *C, ws->splitk, plan->prefix, make_ladder_plane_consts(plan->prefix), stream);
+    st = run_gemm(*ctx, *plan, *A, *B, *C, ws->splitk, plan->prefix, make_ladder_plane_consts(), stream);
   if (st != RNS8_SUCCESS) return st;
   if (exact_wide(plan->desc.semantics)) {
     st = commit_exact_proof(*C, *A, *B, *plan, adm, stream);
@@ -234,7 +234,7 @@ rns8_status gemm_rns_noalloc(rns8_context* ctx, const rns8_plan* plan, const rns
   const hipStream_t stream = pick_stream(*ctx, stream_arg);
   C->device_current = false;
   st = tiled ? run_gemm_tiled(*ctx, *plan, *A, *B, *C, stream)
-             : run_gemm(*ctx, *plan, *A, *B, *C, scratch, plan->prefix, make_ladder_plane_consts(plan->prefix),
+             : run_gemm(*ctx, *plan, *A, *B, *C, scratch, plan->prefix, make_ladder_plane_consts(),
                         stream);
   if (st != RNS8_SUCCESS) return st;
   C->device_current = true;
@@ -282,7 +282,7 @@ rns8_status gemm_native(rns8_context* ctx, const rns8_plan* plan, const T* A, in
   if (!fused_args_ok(f)) return RNS8_UNSUPPORTED_BACKEND;
   if (hipSetDevice(ctx->device_id) != hipSuccess) return RNS8_BACKEND_FAILURE;
   C->device_current = false;
-  const hipError_t e = launch_fused_native(f, make_ladder_plane_consts(plan->prefix), stream);
+  const hipError_t e = launch_fused_native(f, make_ladder_plane_consts(), stream);
   if (e == hipErrorInvalidValue) return RNS8_UNSUPPORTED_BACKEND;
   if (e != hipSuccess) return RNS8_BACKEND_FAILURE;
   C->device_current = true;
@@ -383,7 +383,7 @@ rns8_status gemm_grouped(rns8_context* ctx, const rns8_plan* plan, const rns8_gr
     g.pitch_c = c0.plane_pitch;
     g.nplanes = finite ? 1u : plan->prefix;
     g.slices = plan->splitk_slices;
-    const PlaneConsts consts = finite ? make_single_plane_consts(modulus) : make_ladder_plane_consts(plan->prefix);
+    const PlaneConsts consts = finite ? make_single_plane_consts(modulus) : make_ladder_plane_consts();
     const hipError_t e = launch_gemm_grouped(g, consts, ptrs.data(), task_count, stream);
     st = e == hipSuccess ? RNS8_SUCCESS : e == hipErrorInvalidValue ? RNS8_UNSUPPORTED_BACKEND : RNS8_BACKEND_FAILURE;
   }

@@ -11,25 +11,23 @@
 // only below a workspace limit.
 //
 // Work split: a workgroup owns a 128 x 128 output tile, a pair of planes and
-// one K slice. Its twelve waves run three per SIMD: two converter waves and
-// one MFMA wave each (a single wave issues a VALU instruction only every six
-// or seven cycles, so the conversion needs two waves per SIMD to keep the VALU
-// busy, and the MFMAs issue from a third). Roles:
-//   * conversion: waves 0-3 take A, waves 4-7 take B, and every load is
+// one K slice. Its sixteen waves, four per SIMD, all convert and all multiply
+// (a single wave issues a VALU instruction only every six or seven cycles, so
+// the conversion needs several per SIMD to keep the VALU busy):
+//   * conversion: waves 0-7 take A, waves 8-15 take B, and every load is
 //     coalesced: an A load covers four rows x 32 k (16 lanes per 256-byte row
 //     segment, two k per lane), a B load one k row x 128 columns (two columns
-//     per lane). A lane thus holds two k of eight rows (A) or eight k of two
-//     columns (B). Both roles issue eight 16-byte loads per step; the raw
-//     values of step s+2 are requested while step s is converted. Each lane
-//     reduces its 16 elements for both planes (the pack's arithmetic: two
-//     v_dot4_u32_u8 and a 24-bit quotient, or one dot product when every
-//     element of the wave's step fits in 32 bits) and stores its residues
-//     into the k-contiguous stage (2 bytes per A row, 8 per B column);
-//   * MFMA: wave 8 + q multiplies both planes of the pair over the 64 x 64
-//     quadrant q (2 x 2 blocks of v_mfma_i32_32x32x32_i8 per plane, 128
-//     accumulator registers), one step behind the conversion: the residue
-//     stages are double-buffered and one barrier per step separates a stage's
-//     writers from its readers.
+//     per lane). A lane thus holds two k of four rows (A) or four k of two
+//     columns (B), four 16-byte loads per step; the raw values of step s+1 are
+//     requested while step s is converted. Each lane reduces its 8 elements
+//     for both planes (the pack's arithmetic: two v_dot4_u32_u8 and a 24-bit
+//     quotient, or one dot product when every element of the wave's step fits
+//     in 32 bits) and stores its residues into the k-contiguous stage (2 bytes
+//     per A row, 4 per B column);
+//   * MFMA: wave w multiplies plane w / 8 of the pair over a 64 x 32 slice of
+//     the tile (two v_mfma_i32_32x32x32_i8, 32 accumulator registers), one step
+//     behind the conversion: the residue stages are double-buffered and one
+//     barrier per step separates a stage's writers from its readers.
 // Residue stage layout per plane and operand: [2 k-chunks][128 rows or
 // columns][16 bytes], so both the conversion's stores and the fragment reads
 // (lane l: row or column l & 31 of a block, k-chunk l >> 5) are contiguous

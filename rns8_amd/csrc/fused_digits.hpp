@@ -42,7 +42,8 @@
 // centered residues [slice][row][16 columns x groups] in the workspace; a
 // finalize adds the slices and writes C's planes. Weights and residues take at
 // most kMaxPart bytes each: larger K or m run in parts.
-// (Compiled as part of fused_skinny.hip.)
+// (A header of fused_skinny.hip, not a source: what links the kernels' objects by
+// name, as the CPU fuzzers' build does, needs no further object.)
 #pragma once
 
 #include <algorithm>
@@ -300,7 +301,7 @@ __global__ __launch_bounds__(256) void digits_finalize_kernel(const int8_t* slot
 }
 
 // 16-column groups of the result.
-uint32_t groups_of(uint32_t nplanes, int64_t n) { return (nplanes * static_cast<uint32_t>(n) + 15u) / 16u; }
+inline uint32_t groups_of(uint32_t nplanes, int64_t n) { return (nplanes * static_cast<uint32_t>(n) + 15u) / 16u; }
 
 struct Parts {
   int64_t slices, k_slice;
@@ -309,7 +310,7 @@ struct Parts {
   int64_t part_rows;    // rows whose residues it holds at once
   uint64_t w_bytes, slot_bytes;
 };
-Parts split(int64_t m, int64_t n, int64_t k, uint32_t nplanes) {
+inline Parts split(int64_t m, int64_t n, int64_t k, uint32_t nplanes) {
   Parts p{};
   p.groups = groups_of(nplanes, n);
   const int64_t row_groups = (m + kGroupRows - 1) / kGroupRows;
@@ -330,7 +331,7 @@ Parts split(int64_t m, int64_t n, int64_t k, uint32_t nplanes) {
 
 }  // namespace
 
-bool fused_digits_shape(int64_t m, int64_t n, int64_t k, uint32_t nplanes, FusedShape& out) {
+inline bool fused_digits_shape(int64_t m, int64_t n, int64_t k, uint32_t nplanes, FusedShape& out) {
   if (n <= 0 || n > 16 || m <= 0 || k <= 0 || nplanes == 0 || nplanes > kMaxPrefix) return false;
   if (m >= (int64_t{1} << 31) || k > kMaxK) return false;
   // Where this form is the faster one. Its cost grows with the 16-column groups
@@ -398,7 +399,7 @@ bool fused_digits_shape(int64_t m, int64_t n, int64_t k, uint32_t nplanes, Fused
   return true;
 }
 
-hipError_t launch_fused_digits(const FusedArgs& f, hipStream_t stream) {
+inline hipError_t launch_fused_digits(const FusedArgs& f, hipStream_t stream) {
   const FusedShape& sh = f.shape;
   if (sh.skinny != 2 || f.ldc != 16 || f.n > 16 || f.k > kMaxK || f.lda >= (int64_t{1} << 21)) return hipErrorInvalidValue;
   const Parts p = split(f.m, f.n, f.k, f.nplanes);

@@ -185,9 +185,9 @@ struct TaskPtrs {
 constexpr uint32_t kMaxGroupTasks = 32;
 hipError_t launch_gemm_grouped(const GemmArgs& shape, const PlaneConsts& consts, const TaskPtrs* tasks,
                                uint32_t count, hipStream_t stream);
-// How launch_gemm runs a shape: the kernel (plane_gemm_kernel with 256 or
-// 128 tiles, or the skinny kernel for results at most 16 columns wide) and
-// the K split. A split covers the whole K in slices of at most 65536, each
+// How launch_gemm runs a shape: the kernel (plane_gemm_kernel with one of five
+// tiles, or the skinny kernel for results at most 16 columns wide) and the K
+// split. A split covers the whole K in slices of at most 65536, each
 // writing its centered residues to the int8 workspace, and a finalize adds
 // them; unsplit products with K beyond 65536 run as accumulating launches.
 enum class GemmTile : uint32_t { k256x256, k256x128, k128x256, k128x128, k64x64, kSkinny };

@@ -31,11 +31,13 @@ constexpr int64_t kSafeKBlock = 65536;
 // Centering: with H = floor(m/2), centered(x) = ((x + H) mod m) - H equals the
 // reference rule "r >= (m+1)/2 ? r - m : r" (cpu_reference.cpp:26-32) for
 // every m >= 2. H is folded into the additive offsets below.
+
 // Start value of the plane GEMM's accumulators: a GEMM sum is at most 2^30 in
 // magnitude (65536 products of 2^14) plus a carried residue, so sum + bias
 // stays inside [0, 2^32); 0x40800000 is the bit pattern of 4.0f, which an MFMA
 // takes as an inline C operand, and 0 modulo 256.
 constexpr uint32_t kGemmAccBias = 0x40800000u;
+
 struct ModulusConsts {
   uint32_t m;
   uint32_t half;    // H = floor(m/2)
@@ -143,7 +145,7 @@ struct PlaneConsts {
   uint32_t modulus;  // 0: plane p has modulus kLadder[p]
 };
 
-inline PlaneConsts make_ladder_plane_consts(uint32_t) { return PlaneConsts{0}; }
+inline PlaneConsts make_ladder_plane_consts() { return PlaneConsts{0}; }
 inline PlaneConsts make_single_plane_consts(uint32_t modulus) { return PlaneConsts{modulus}; }
 
 // The table: the ladder's kMaxPrefix moduli, then every modulus 0 .. 256 (0

@@ -55,7 +55,7 @@ RESIDUE_FASTER = [
     # five and six planes
     (1160, 10, 6968, 6), (5748, 5, 6620, 5), (53, 5, 53387, 6),
     # many groups for the planes
-    (8192, 8, 8192, 9), (200, 16, 3000, 18),
+    (8192, 8, 8192, 9), (200, 16, 3000, 18), (8, 8, 1 << 20, 9),
 ]
 DIGITS_FASTER = [
     (8192, 1, 8192, 9), (8192, 7, 8192, 9), (2000, 7, 1000, 9), (128, 7, 256, 9), (200, 4, 20000, 20), (512, 3, 512, 5),
