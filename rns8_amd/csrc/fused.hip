@@ -477,7 +477,6 @@ bool fused_args_ok(const FusedArgs& a) {
 
 hipError_t launch_fused_native(const FusedArgs& a, const PlaneConsts& consts, hipStream_t stream) {
   if (!fused_args_ok(a)) return hipErrorInvalidValue;
-  if (a.shape.skinny == 2) return digits::launch_fused_digits(a, stream);
   if (a.shape.skinny) return launch_fused_skinny(a, consts, stream);
   const uint32_t tiles_n = static_cast<uint32_t>((a.n + kTileN - 1) / kTileN);
   const uint32_t tiles = static_cast<uint32_t>((a.m + kTileM - 1) / kTileM) * tiles_n;

@@ -391,6 +391,7 @@ bool fused_skinny_shape(int64_t m, int64_t n, int64_t k, uint32_t nplanes, Fused
 
 hipError_t launch_fused_skinny(const FusedArgs& f, const PlaneConsts& consts, hipStream_t stream) {
   const FusedShape& sh = f.shape;
+  if (sh.skinny == 2) return digits::launch_fused_digits(f, stream);
   if (sh.skinny != 1 || f.ldc != 16 || f.n > 16 || f.k > kMaxK || f.lda >= (int64_t{1} << 21)) return hipErrorInvalidValue;
   const int64_t kp = kp_of(f.k);
   const bool sgn = f.kind == NativeKind::I64;

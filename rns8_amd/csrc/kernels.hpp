@@ -149,15 +149,9 @@ struct FusedArgs {
 // otherwise, before enqueuing anything).
 bool fused_args_ok(const FusedArgs& args);
 hipError_t launch_fused_native(const FusedArgs& args, const PlaneConsts& consts, hipStream_t stream);
-// The skinny form (shape.skinny), called by launch_fused_native once the
-// arguments are checked.
+// The skinny forms (shape.skinny 1 and 2), called by launch_fused_native once
+// the arguments are checked.
 hipError_t launch_fused_skinny(const FusedArgs& args, const PlaneConsts& consts, hipStream_t stream);
-// The digit form (shape.skinny == 2, fused_digits.hpp) and which products
-// among the skinny form's run it.
-namespace digits {
-hipError_t launch_fused_digits(const FusedArgs& args, hipStream_t stream);
-bool fused_digits_shape(int64_t m, int64_t n, int64_t k, uint32_t nplanes, FusedShape& out);
-}  // namespace digits
 // Per-tile schedules: `units` edge x edge tile-planes (edge 256 or 128) from a
 // device list of two words each, (plane << 24 | tile row) and (quadrant mask
 // << 24 | tile column); bit q = 2 * (row half) + (column half) of the mask
