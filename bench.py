@@ -392,19 +392,21 @@ def main() -> int:
     traffic_kernels, traffic_workload = ["plane_gemm_kernel"], args.config
     if fused:
         # pack and GEMM in one pass: the native operands are read (8 bytes per
-        # element) and the C planes written; HBM bounds it for tall-skinny shapes
-        # results at most 16 columns wide take the skinny form (B's planes
-        # first, then A converted in registers) while its workspace fits 256 MiB
-        skinny_form = N <= 16 and P * 16 * ((K + 63) // 64 * 64) <= (256 << 20)
-        kernel = ("pack_bt_kernel + fused_skinny_kernel<Signed,G,First256> + residue_finalize_kernel" if skinny_form
-                  else "fused_native_kernel<Signed,NP> + residue_finalize_kernel")
+        # element) and the C planes written; HBM bounds it for tall-skinny
+        # shapes. Results at most 16 columns wide run one of two narrow forms
+        # (tests/test_dispatch.py holds which): B's digit weights first and A's
+        # bytes multiplied as they are, or B's planes first and A converted in
+        # registers; wider ones the tile form
+        traffic_kernels = {"gemv1": ["digit_weights_kernel", "fused_digits_kernel", "digits_finalize_kernel"],
+                           "gemv8": ["pack_bt_kernel", "fused_skinny_kernel", "residue_finalize_kernel"],
+                           "small64": ["pack_bt_kernel", "fused_skinny_kernel", "residue_finalize_kernel"]}.get(
+                               args.config, ["fused_native_kernel", "residue_finalize_kernel"])
+        kernel = " + ".join(traffic_kernels)
         workload = workload.replace("pack+GEMM", "fused pack+GEMM")
         gemm_bytes = 8 * K * (M + N) + P * M * N
         gbs = gemm_bytes / ((stage[0] + stage[1] + stage[2]) * 1e-3) / 1e9
         roofline = {"bound": "hbm", "kernel": kernel, "achieved": round(gbs, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
                     "frac": round(gbs / PEAK_HBM_GBS, 4), "per_launch_bytes": gemm_bytes}
-        traffic_kernels = (["pack_bt_kernel", "fused_skinny_kernel", "residue_finalize_kernel"] if skinny_form
-                           else ["fused_native_kernel", "residue_finalize_kernel"])
     elif args.config in SKINNY:
         # at most 16 columns: the GEMM reads A's planes once and B's (padded
         # to 16 columns) once, so HBM bounds it
