@@ -13,6 +13,8 @@ def test_bench_reads_committed_traffic():
     import bench
 
     assert bench.traffic_from_profiles("plane_gemm_kernel", "c3") > 0
+    assert bench.traffic_from_profiles(["digit_weights_kernel", "fused_digits_kernel", "digits_finalize_kernel"],
+                                       "gemv1") > 0
     assert bench.traffic_from_profiles(["pack_bt_kernel", "fused_skinny_kernel", "residue_finalize_kernel"],
                                        "gemv1") > 0
     assert bench.traffic_from_profiles(["skinny_gemm_kernel", "residue_finalize_kernel"], "gemv1_packed") > 0
